@@ -40,6 +40,7 @@ MFMA_VGPR = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 SOURCES = [
     ("csrc/ntt.hip", True, []),
     ("csrc/bconv.hip", True, MFMA_VGPR),
+    ("csrc/switch_cols.hip", True, MFMA_VGPR),
     ("csrc/elementwise.hip", True, []),
     ("csrc/hmult_noalloc.hip", True, []),
     ("host/device_tables.cpp", False, []),

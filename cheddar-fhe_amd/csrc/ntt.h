@@ -60,6 +60,9 @@ struct NttArgs {
   // centred source limb src + z * src_pstride, times its cst[l] (a
   // one-source BConv fused into the transform's first round)
   int src_bcast;
+  // row passes only: the input (forward) or output (inverse) is
+  // column-blocked and apart from the other side
+  int blocked;
 };
 
 // Fused ModUp row pass + evaluation-key inner product (PAccum) + CAccum for
@@ -85,6 +88,9 @@ hipError_t launch_ntt_inv(const NttArgs &a, int num_limbs, int num_polys,
 hipError_t launch_ntt_fwd_cols(const NttArgs &a, int num_limbs, int num_z,
                                hipStream_t s);
 hipError_t launch_ntt_fwd_rows(const NttArgs &a, int num_limbs, int num_z,
+                               int epilogue, hipStream_t s);
+// the inverse's first pass alone
+hipError_t launch_ntt_inv_rows(const NttArgs &a, int num_limbs, int num_polys,
                                hipStream_t s);
 
 }  // namespace chd

@@ -194,15 +194,39 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Coalesced tile layout of the row passes: a workgroup owns kTileRows
-// consecutive rows (16 KiB contiguous); in store round v (0..3) thread t owns
-// the 16 bytes at tile offset 16 (t + 256 v), i.e. tile elements
-// 4 (t + 256 v) .. + 3.
-__device__ __forceinline__ uint32_t tile_byte(int tile) {
-  return static_cast<uint32_t>(tile) * (kTileRows * kCols * 4u);
+// Row tile of a row pass: kTileRows rows of a limb, tile blockIdx.x. Row r of
+// it is row 16 blockIdx.x + r, or, with column-blocked data on one side,
+// row 16 r + blockIdx.x.
+__device__ __forceinline__ int tile_row(bool blocked, int r) {
+  return blocked ? kTileRows * r + static_cast<int>(blockIdx.x)
+                 : static_cast<int>(blockIdx.x) * kTileRows + r;
 }
-__device__ __forceinline__ uint32_t tile_lane_byte(int v) {
-  return (threadIdx.x + 256u * v) * 16u;
+// Coalesced access to the tile in the usual order: in round v (0..3) thread t
+// owns tile elements 4 (t + 256 v) .. + 3, so a wave moves one row (1 KiB).
+// Byte offset of the tile in its limb, and of round v in the tile:
+__device__ __forceinline__ uint32_t tile_byte(bool blocked) {
+  return blockIdx.x * (blocked ? kCols * 4u : kTileRows * kCols * 4u);
+}
+__device__ __forceinline__ uint32_t tile_lane_byte(bool blocked, int v) {
+  return blocked ? (threadIdx.x >> 6) * (kTileRows * kCols * 4u) +
+                       (threadIdx.x & 63) * 16u +
+                       v * (4u * kTileRows * kCols * 4u)
+                 : (threadIdx.x + 256u * v) * 16u;
+}
+// Column-blocked limbs (between a base switch's row passes and its column
+// stage): column col of row 16 r + t at word
+//   ((col >> 2) * 256 + 16 t + r) * 4 + (col & 3),
+// so that tile t is 64 pieces of 256 bytes (4 columns of its 16 rows) and
+// the column stage's lane r, which needs rows 16 r .. 16 r + 15, sits next to
+// lane r + 1's words. Word of column c + 16 k of the tile's row r:
+__device__ __forceinline__ uint32_t blocked_word(int r, int c) {
+  return (c >> 2) * 1024u + (blockIdx.x * kTileRows + r) * 4u + (c & 3);
+}
+constexpr int kBlockedStep = 4096;  // words from column c to c + 16
+// in store round v thread t owns the 16 bytes of row t % 16, columns
+// 4 (t / 16 + 16 v) .. + 3
+__device__ __forceinline__ uint32_t blocked_byte(int v) {
+  return 4u * blocked_word(threadIdx.x & 15, 4 * ((threadIdx.x >> 4) + 16 * v));
 }
 
 // base of polynomial z: explicit list or base + z * stride
@@ -295,6 +319,16 @@ __device__ __forceinline__ u32x4 tile_lds4(const uint32_t *xt, int v) {
   const int e = 4 * (threadIdx.x + 256 * v);
   const uint32_t *p = xt + (e >> 8) * kRowPad;
   const int cc = e & 255;
+  u32x4 o;
+#pragma unroll
+  for (int j = 0; j < 4; j++) o[j] = p[pidx(cc + j)];
+  return o;
+}
+
+// the 4 words of store round v of a column-blocked tile (blocked_byte)
+__device__ __forceinline__ u32x4 blocked_lds4(const uint32_t *xt, int v) {
+  const uint32_t *p = xt + (threadIdx.x & 15) * kRowPad;
+  const int cc = 4 * ((threadIdx.x >> 4) + 16 * v);
   u32x4 o;
 #pragma unroll
   for (int j = 0; j < 4; j++) o[j] = p[pidx(cc + j)];
@@ -480,7 +514,7 @@ __global__ __launch_bounds__(512) void ntt_fwd_cols(NttArgs a) {
 
 // forward, row pass: stages 8..15 (in place on dst) + epilogue
 // grid (kRows / kTileRows, limbs, polys), block 256
-template <int kEpi, bool kLazy>
+template <int kEpi, bool kLazy, bool kBlocked>
 __device__ __forceinline__ void fwd_rows_body(const NttArgs &a, const Limb &lb,
                                               uint32_t (&xin)[16], uint32_t q,
                                               uint32_t qinv, uint32_t *dst,
@@ -492,7 +526,7 @@ __device__ __forceinline__ void fwd_rows_body(const NttArgs &a, const Limb &lb,
   const uint32_t *tw = a.tab.tw + (static_cast<size_t>(lb.ti) << kLogN);
   const int c = threadIdx.x & 15;
   const int r = threadIdx.x >> 4;
-  const int row = blockIdx.x * kTileRows + r;
+  const int row = tile_row(kBlocked, r);
   T *xr = reinterpret_cast<T *>(xch) + r * kRowPad;
   uint32_t w1[15], w2[15];
 #pragma unroll
@@ -543,7 +577,7 @@ __device__ __forceinline__ void fwd_rows_body(const NttArgs &a, const Limb &lb,
   for (int k = 0; k < 16; k++) xu[pidx(16 * c + k)] = ar.canon_fwd(x[k]);
   __syncthreads();
   const uint32_t *xt = reinterpret_cast<const uint32_t *>(xch);
-  char *tile = reinterpret_cast<char *>(dst) + tile_byte(blockIdx.x);
+  char *tile = reinterpret_cast<char *>(dst) + tile_byte(kBlocked);
   [[maybe_unused]] const int32_t qs = static_cast<int32_t>(q);
   [[maybe_unused]] int32_t c2 = 0, c2q = 0;
   if constexpr (kEpi == kEpiModDown) {
@@ -563,11 +597,12 @@ __device__ __forceinline__ void fwd_rows_body(const NttArgs &a, const Limb &lb,
         o[j] = static_cast<uint32_t>(norm(mont(d, c2, c2q, qs), qs));
       }
     }
-    st_nt<u32x4>(tile, tile_lane_byte(v), o);
+    st_nt<u32x4>(tile, tile_lane_byte(kBlocked, v), o);
   }
 }
 
-template <int kEpi>
+// kBlocked: the input is column-blocked and apart from dst
+template <int kEpi, bool kBlocked>
 __global__ __launch_bounds__(256) void ntt_fwd_rows(NttArgs a) {
   __shared__ int32_t xch[kTileRows * kRowPad];
   LimbMap m = a.map;
@@ -583,12 +618,21 @@ __global__ __launch_bounds__(256) void ntt_fwd_rows(NttArgs a) {
   uint32_t *dst =
       poly_dst(a, blockIdx.z) + (static_cast<size_t>(lb.l) << kLogN);
   const int c = threadIdx.x & 15;
-  const uint32_t rbase =
-      static_cast<uint32_t>((blockIdx.x * kTileRows + (threadIdx.x >> 4)) *
-                            kCols) * 4u;
+  const int r = threadIdx.x >> 4;
   uint32_t x[16];
+  if constexpr (kBlocked) {
+    const uint32_t *src = a.src + blockIdx.z * a.src_pstride +
+                          (static_cast<size_t>(lb.l) << kLogN);
+    const uint32_t off = 4u * blocked_word(r, c);
 #pragma unroll
-  for (int k = 0; k < 16; k++) x[k] = ld_nt<uint32_t>(dst, rbase + (c + 16 * k) * 4u);
+    for (int k = 0; k < 16; k++)
+      x[k] = ld_at<uint32_t>(src + kBlockedStep * k, off);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 16; k++)
+      x[k] = ld_nt<uint32_t>(
+          dst, tile_row(false, r) * (kCols * 4u) + (c + 16 * k) * 4u);
+  }
   // ModDown epilogue operand: src2 at this thread's 16 output words of the
   // coalesced store layout (zero outside [src2_lo, src2_hi)), loaded with the
   // data so their latency hides behind the butterflies
@@ -597,11 +641,11 @@ __global__ __launch_bounds__(256) void ntt_fwd_rows(NttArgs a) {
     if (lb.l >= a.src2_lo && lb.l < a.src2_hi) {
       const uint32_t *s2p = a.src2 + blockIdx.z * a.src2_pstride +
                             (static_cast<size_t>(lb.l - a.src2_lo) << kLogN);
-      const char *s2t = reinterpret_cast<const char *>(s2p) +
-                        tile_byte(blockIdx.x);
+      const char *s2t =
+          reinterpret_cast<const char *>(s2p) + tile_byte(kBlocked);
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        const uint4 t = ld_nt<uint4>(s2t, tile_lane_byte(v));
+        const uint4 t = ld_nt<uint4>(s2t, tile_lane_byte(kBlocked, v));
         s2v[4 * v] = t.x;
         s2v[4 * v + 1] = t.y;
         s2v[4 * v + 2] = t.z;
@@ -624,19 +668,19 @@ __global__ __launch_bounds__(256) void ntt_fwd_rows(NttArgs a) {
     }
   }
   if (q < (1u << 30))
-    fwd_rows_body<kEpi, true>(a, lb, x, q, qinv, dst, xch, s2v);
+    fwd_rows_body<kEpi, true, kBlocked>(a, lb, x, q, qinv, dst, xch, s2v);
   else
-    fwd_rows_body<kEpi, false>(a, lb, x, q, qinv, dst, xch, s2v);
+    fwd_rows_body<kEpi, false, kBlocked>(a, lb, x, q, qinv, dst, xch, s2v);
 }
 
-// twiddles of the inverse row pass for this thread of a 16-row tile (row
-// tile blockIdx.x): w2 for stages 15..12 (columns 16c + k), w1 for stages
-// 11..8 (the row's)
+// twiddles of the inverse row pass for this thread of a row tile: w2 for
+// stages 15..12 (columns 16c + k), w1 for stages 11..8 (the row's)
 __device__ __forceinline__ void inv_row_twiddles(const uint32_t *itw,
+                                                 bool blocked,
                                                  uint32_t (&w1)[15],
                                                  uint32_t (&w2)[15]) {
   const int c = threadIdx.x & 15;
-  const int row = blockIdx.x * kTileRows + (threadIdx.x >> 4);
+  const int row = tile_row(blocked, threadIdx.x >> 4);
 #pragma unroll
   for (int s = 0, i = 0; s < 4; s++)
 #pragma unroll
@@ -654,7 +698,7 @@ __device__ __forceinline__ void inv_rows_body(const uint32_t (&w1)[15],
                                               const uint32_t (&w2)[15],
                                               uint32_t (&xin)[16], uint32_t q,
                                               uint32_t qinv, uint32_t *dst,
-                                              int32_t *xch) {
+                                              int32_t *xch, bool blocked) {
   using A = Arith<kLazy>;
   using T = typename A::T;
   const A ar(q, qinv);
@@ -697,11 +741,21 @@ __device__ __forceinline__ void inv_rows_body(const uint32_t (&w1)[15],
   for (int k = 0; k < 16; k++) xr[pidx(c + 16 * k)] = x[k];
   __syncthreads();
   const uint32_t *xt = reinterpret_cast<const uint32_t *>(xch);
-  char *tile = reinterpret_cast<char *>(dst) + tile_byte(blockIdx.x);
+  if (blocked) {
+    // the column stage reads it right away: default caching
 #pragma unroll
-  for (int v = 0; v < 4; v++) st_nt<u32x4>(tile, tile_lane_byte(v), tile_lds4(xt, v));
+    for (int v = 0; v < 4; v++)
+      st_at<u32x4>(dst, blocked_byte(v), blocked_lds4(xt, v));
+    return;
+  }
+  char *tile = reinterpret_cast<char *>(dst) + tile_byte(false);
+#pragma unroll
+  for (int v = 0; v < 4; v++)
+    st_nt<u32x4>(tile, tile_lane_byte(false, v), tile_lds4(xt, v));
 }
 
+// kBlocked: the output is column-blocked and apart from src
+template <bool kBlocked>
 __global__ __launch_bounds__(256) void ntt_inv_rows(NttArgs a) {
   __shared__ int32_t xch[kTileRows * kRowPad];
   const Limb lb = decode(a.map, blockIdx.y);
@@ -710,18 +764,21 @@ __global__ __launch_bounds__(256) void ntt_inv_rows(NttArgs a) {
   uint32_t *dst =
       poly_dst(a, blockIdx.z) + (static_cast<size_t>(lb.l) << kLogN);
   const int c = threadIdx.x & 15;
-  // the tile (16 contiguous rows) is read with coalesced 16-byte loads and
+  // the tile is read with coalesced 16-byte loads and
   // regrouped through LDS into this thread's 16 consecutive columns (1 us
   // faster at 64 limbs than 16-byte loads at a 64-byte stride, measured)
-  const char *tile = reinterpret_cast<const char *>(src) + tile_byte(blockIdx.x);
+  const char *tile =
+      reinterpret_cast<const char *>(src) + tile_byte(kBlocked);
   u32x4 v4[4];
 #pragma unroll
-  for (int v = 0; v < 4; v++) v4[v] = ld_at<u32x4>(tile, tile_lane_byte(v));
+  for (int v = 0; v < 4; v++)
+    v4[v] = ld_at<u32x4>(tile, tile_lane_byte(kBlocked, v));
   // twiddles of both half-passes, requested with the tile so their latency
   // hides behind its load and the LDS regrouping (stages 15..12: columns
   // 16c + k; stages 11..8: the row's)
   uint32_t w1[15], w2[15];
-  inv_row_twiddles(a.tab.itw + (static_cast<size_t>(lb.ti) << kLogN), w1, w2);
+  inv_row_twiddles(a.tab.itw + (static_cast<size_t>(lb.ti) << kLogN),
+                   kBlocked, w1, w2);
   const uint32_t q = a.tab.q[lb.ti];
   const uint32_t qinv = static_cast<uint32_t>(a.tab.qinv[lb.ti]);
   if (a.src_mul != nullptr) {
@@ -729,10 +786,10 @@ __global__ __launch_bounds__(256) void ntt_inv_rows(NttArgs a) {
     const char *sm = reinterpret_cast<const char *>(
                          a.src_mul + blockIdx.z * a.src_pstride +
                          (static_cast<size_t>(lb.sl) << kLogN)) +
-                     tile_byte(blockIdx.x);
+                     tile_byte(kBlocked);
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      const u32x4 y = ld_at<u32x4>(sm, tile_lane_byte(v));
+      const u32x4 y = ld_at<u32x4>(sm, tile_lane_byte(kBlocked, v));
 #pragma unroll
       for (int j = 0; j < 4; j++)
         v4[v][j] = mont_mul(static_cast<int32_t>(v4[v][j]),
@@ -755,9 +812,9 @@ __global__ __launch_bounds__(256) void ntt_inv_rows(NttArgs a) {
 #pragma unroll
   for (int k = 0; k < 16; k++) x[k] = xr[pidx(16 * c + k)];
   if (q < (1u << 30))
-    inv_rows_body<true>(w1, w2, x, q, qinv, dst, xch);
+    inv_rows_body<true>(w1, w2, x, q, qinv, dst, xch, kBlocked);
   else
-    inv_rows_body<false>(w1, w2, x, q, qinv, dst, xch);
+    inv_rows_body<false>(w1, w2, x, q, qinv, dst, xch, kBlocked);
 }
 
 // inverse, column pass: GS stages 7..0 (in place on dst) + constant epilogue
@@ -869,7 +926,7 @@ __device__ __forceinline__ void keyacc_body(const chd_keyacc_args &a,
   const uint32_t *tw = tab.tw + (static_cast<size_t>(ti) << kLogN);
   const int c = threadIdx.x & 15;
   const int r = threadIdx.x >> 4;
-  const int row = blockIdx.x * kTileRows + r;
+  const int row = tile_row(a.blocked, r);
   const uint32_t rbase = static_cast<uint32_t>(row * kCols) * 4u;
   // Element ownership of the products: register k = 4v + j holds column
   // 4c + 64v + j of the thread's row, so the 16 threads of a row move 256
@@ -878,6 +935,10 @@ __device__ __forceinline__ void keyacc_body(const chd_keyacc_args &a,
   // wave-level fence.
   const uint32_t obase = rbase + 16u * c;
   T *xr = reinterpret_cast<T *>(xch) + r * kRowPad;
+  // column c + 16 k of the thread's row in modup (row-major or blocked)
+  const uint32_t ubase =
+      a.blocked ? 4u * blocked_word(r, c) : rbase + 4u * c;
+  const int ustep = a.blocked ? kBlockedStep : 16;  // words
   // twiddles are (re)loaded inside each group's row pass (cache hits after
   // the first group) instead of living in 30 registers across the loop
   const size_t loff = static_cast<size_t>(l) << kLogN;
@@ -902,7 +963,8 @@ __device__ __forceinline__ void keyacc_body(const chd_keyacc_args &a,
   const bool intt_here = a.intt_b != nullptr && l >= a.intt_lo;
   uint32_t iw1[15], iw2[15];
   if (intt_here)
-    inv_row_twiddles(tab.itw + (static_cast<size_t>(ti) << kLogN), iw1, iw2);
+    inv_row_twiddles(tab.itw + (static_cast<size_t>(ti) << kLogN), a.blocked,
+                     iw1, iw2);
   int nprod = 0;        // products in sb / sa (uniform)
   bool folded = false;  // accb / acca hold earlier products
   auto fold = [&]() {
@@ -986,7 +1048,7 @@ __device__ __forceinline__ void keyacc_body(const chd_keyacc_args &a,
       T x[16];
 #pragma unroll
       for (int k = 0; k < 16; k++)
-        x[k] = static_cast<T>(ld_at<uint32_t>(src, rbase + (c + 16 * k) * 4u));
+        x[k] = static_cast<T>(ld_at<uint32_t>(src + k * ustep, ubase));
 #pragma unroll
       for (int s = 0, i = 0; s < 4; s++) {
         const int h = 8 >> s;
@@ -1100,10 +1162,12 @@ __device__ __forceinline__ void keyacc_body(const chd_keyacc_args &a,
       for (int k = 0; k < 16; k++) acc[k] = xr[pidx(16 * c + k)];
     };
     to_rows(accb);
-    inv_rows_body<kLazy>(w1, w2, accb, q, qinv, a.intt_b + ioff, xch);
+    inv_rows_body<kLazy>(w1, w2, accb, q, qinv, a.intt_b + ioff, xch,
+                         a.blocked != 0);
     __syncthreads();  // the first polynomial's store reads cross rows
     to_rows(acca);
-    inv_rows_body<kLazy>(w1, w2, acca, q, qinv, a.intt_a + ioff, xch);
+    inv_rows_body<kLazy>(w1, w2, acca, q, qinv, a.intt_a + ioff, xch,
+                         a.blocked != 0);
     return;
   }
   uint32_t *ob = a.acc_b + loff;
@@ -1826,10 +1890,17 @@ hipError_t launch_ntt_fwd_cols(const NttArgs &a, int num_limbs, int num_z,
 }
 
 hipError_t launch_ntt_fwd_rows(const NttArgs &a, int num_limbs, int num_z,
-                               hipStream_t s) {
+                               int epilogue, hipStream_t s) {
   if (num_limbs <= 0 || num_z <= 0) return hipSuccess;
   dim3 gr(kRows / kTileRows, num_limbs, num_z);
-  hipLaunchKernelGGL(ntt_fwd_rows<kEpiStore>, gr, dim3(256), 0, s, a);
+  if (epilogue == kEpiModDown && a.blocked)
+    hipLaunchKernelGGL((ntt_fwd_rows<kEpiModDown, true>), gr, dim3(256), 0, s, a);
+  else if (epilogue == kEpiModDown)
+    hipLaunchKernelGGL((ntt_fwd_rows<kEpiModDown, false>), gr, dim3(256), 0, s, a);
+  else if (a.blocked)
+    hipLaunchKernelGGL((ntt_fwd_rows<kEpiStore, true>), gr, dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((ntt_fwd_rows<kEpiStore, false>), gr, dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
@@ -1867,18 +1938,13 @@ hipError_t launch_ntt_fwd(const NttArgs &a, int num_limbs, int num_polys,
     return hipGetLastError();
   }
   dim3 gc(kCols / kTileCols, num_limbs, num_polys);
-  dim3 gr(kRows / kTileRows, num_limbs, num_polys);
   if (pre_const)
     hipLaunchKernelGGL(ntt_fwd_cols<true>, gc, dim3(512), 0, s, a);
   else
     hipLaunchKernelGGL(ntt_fwd_cols<false>, gc, dim3(512), 0, s, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  if (epilogue == kEpiModDown)
-    hipLaunchKernelGGL(ntt_fwd_rows<kEpiModDown>, gr, dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL(ntt_fwd_rows<kEpiStore>, gr, dim3(256), 0, s, a);
-  return hipGetLastError();
+  return launch_ntt_fwd_rows(a, num_limbs, num_polys, epilogue, s);
 }
 
 hipError_t launch_ntt_inv_cols(const NttArgs &a, int num_limbs, int num_polys,
@@ -1888,6 +1954,17 @@ hipError_t launch_ntt_inv_cols(const NttArgs &a, int num_limbs, int num_polys,
     hipLaunchKernelGGL(ntt_inv_cols<kEpiConstCentre>, gc, dim3(512), 0, s, a);
   else
     hipLaunchKernelGGL(ntt_inv_cols<kEpiConst>, gc, dim3(512), 0, s, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_ntt_inv_rows(const NttArgs &a, int num_limbs, int num_polys,
+                               hipStream_t s) {
+  if (num_limbs <= 0 || num_polys <= 0) return hipSuccess;
+  dim3 gr(kRows / kTileRows, num_limbs, num_polys);
+  if (a.blocked)
+    hipLaunchKernelGGL(ntt_inv_rows<true>, gr, dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL(ntt_inv_rows<false>, gr, dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
@@ -1910,9 +1987,7 @@ hipError_t launch_ntt_inv(const NttArgs &a, int num_limbs, int num_polys,
                          num_limbs, items);
     return hipGetLastError();
   }
-  dim3 gr(kRows / kTileRows, num_limbs, num_polys);
-  hipLaunchKernelGGL(ntt_inv_rows, gr, dim3(256), 0, s, a);
-  hipError_t e = hipGetLastError();
+  hipError_t e = launch_ntt_inv_rows(a, num_limbs, num_polys, s);
   if (e != hipSuccess) return e;
   // the column pass works in place on dst
   NttArgs b = a;
@@ -2161,6 +2236,38 @@ extern "C" int chd_k_ntt_inv_mul(const chd_tables *t, const chd_limb_map *m,
                         centre, stream);
 }
 
+extern "C" int chd_k_ntt_inv_rows(const chd_tables *t, const chd_limb_map *m,
+                                  uint32_t *dst, long long dst_pstride,
+                                  const uint32_t *src, const uint32_t *src_mul,
+                                  long long src_pstride, int num_limbs,
+                                  int num_polys, void *stream) {
+  if (!t || !m || !dst || !src || num_limbs < 0 || num_polys < 0)
+    return set_error(CHD_ERR_ARG, "chd_k_ntt_inv_rows: invalid argument");
+  // the output is in another order than the input: no overlap at all
+  for (const uint32_t *p : {src, src_mul})
+    if (p != nullptr &&
+        !sets_disjoint(p, src_pstride, num_polys,
+                       span_limbs(num_limbs, *m, true), dst, dst_pstride,
+                       num_polys, span_limbs(num_limbs, *m, false)))
+      return set_error(CHD_ERR_ARG,
+                       "chd_k_ntt_inv_rows: a source overlaps the destination");
+  NttArgs a{};
+  a.src = src;
+  a.src_mul = src_mul;
+  a.dst = dst;
+  a.src_pstride = src_pstride;
+  a.dst_pstride = dst_pstride;
+  a.map = *m;
+  a.tab = *t;
+  a.blocked = 1;
+  hipError_t e = launch_ntt_inv_rows(a, num_limbs, num_polys,
+                                     static_cast<hipStream_t>(stream));
+  if (e != hipSuccess)
+    return set_error(CHD_ERR_HIP, std::string("chd_k_ntt_inv_rows: ") +
+                                      hipGetErrorString(e));
+  return 0;
+}
+
 extern "C" int chd_k_ntt_fwd_groups(const chd_tables *t, const chd_limb_map *m,
                                     uint32_t *modup, long long group_stride,
                                     int num_groups, int alpha, int group_shift,
@@ -2200,9 +2307,48 @@ extern "C" int chd_k_ntt_fwd_groups_batch(
   const int nz = num_groups * num_inputs;
   hipError_t e = launch_ntt_fwd_cols(a, group_limbs - min_skip, nz, s);
   if (e == hipSuccess && with_rows)
-    e = launch_ntt_fwd_rows(a, group_limbs - min_skip, nz, s);
+    e = launch_ntt_fwd_rows(a, group_limbs - min_skip, nz, kEpiStore, s);
   if (e != hipSuccess)
     return set_error(CHD_ERR_HIP, std::string("chd_k_ntt_fwd_groups: ") +
+                                      hipGetErrorString(e));
+  return 0;
+}
+
+extern "C" int chd_k_ntt_fwd_rows_groups(
+    const chd_tables *t, const chd_limb_map *m, uint32_t *const *dst,
+    const uint32_t *src, long long group_stride, int num_groups, int alpha,
+    int group_shift, int group_limbs, void *stream) {
+  if (!t || !m || !dst || !src || group_limbs < m->num_q ||
+      num_groups > CHD_MAX_JOBS ||
+      !groups_valid(num_groups, alpha, group_shift, m->num_q))
+    return set_error(CHD_ERR_ARG,
+                     "chd_k_ntt_fwd_rows_groups: invalid argument");
+  NttArgs a{};
+  a.src = src;
+  a.src_pstride = group_stride;
+  a.map = *m;
+  a.map.src_gap = 0;
+  a.tab = *t;
+  a.group_alpha = alpha;
+  a.group_shift = group_shift;
+  a.group_limbs = group_limbs;
+  a.blocked = 1;
+  int min_skip = alpha;
+  for (int g = 0; g < num_groups; g++) {
+    if (!dst[g] || !sets_disjoint(src, group_stride, num_groups, group_limbs,
+                                  dst[g], 0, 1, group_limbs))
+      return set_error(CHD_ERR_ARG,
+                       "chd_k_ntt_fwd_rows_groups: null destination, or it "
+                       "overlaps the source");
+    a.dst_list[g] = dst[g];
+    min_skip = std::min(min_skip, group_hi(g, alpha, group_shift, m->num_q) -
+                                      group_lo(g, alpha, group_shift));
+  }
+  hipError_t e =
+      launch_ntt_fwd_rows(a, group_limbs - min_skip, num_groups, kEpiStore,
+                          static_cast<hipStream_t>(stream));
+  if (e != hipSuccess)
+    return set_error(CHD_ERR_HIP, std::string("chd_k_ntt_fwd_rows_groups: ") +
                                       hipGetErrorString(e));
   return 0;
 }
@@ -2294,6 +2440,47 @@ int moddown_multi_args(const char *who, const chd_tables *t,
 }
 }  // namespace
 
+namespace {
+// no polynomial of a separate ModDown source overlaps a destination
+bool moddown_src_disjoint(const NttArgs &a, const uint32_t *src,
+                          long long src_pstride, int num_polys,
+                          int num_limbs) {
+  for (int p = 0; p < num_polys; p++)
+    if (!sets_disjoint(src, src_pstride, num_polys,
+                       span_limbs(num_limbs, a.map, true), a.dst_list[p], 0, 1,
+                       span_limbs(num_limbs, a.map, false)))
+      return false;
+  return true;
+}
+}  // namespace
+
+extern "C" int chd_k_ntt_fwd_rows_moddown(
+    const chd_tables *t, const chd_limb_map *m, uint32_t *const *dst,
+    int num_polys, int num_limbs, const uint32_t *src, long long src_pstride,
+    const uint32_t *src2, long long src2_pstride, int src2_lo, int src2_hi,
+    const uint32_t *inv_prod, const uint32_t *pad, void *stream) {
+  const char *who = "chd_k_ntt_fwd_rows_moddown";
+  if (!src)
+    return set_error(CHD_ERR_ARG, std::string(who) + ": invalid argument");
+  NttArgs a;
+  if (int st = moddown_multi_args(who, t, m, dst, num_polys, num_limbs, src2,
+                                  src2_pstride, src2_lo, src2_hi, inv_prod,
+                                  pad, &a))
+    return st;
+  if (!moddown_src_disjoint(a, src, src_pstride, num_polys, num_limbs))
+    return set_error(CHD_ERR_ARG,
+                     std::string(who) + ": source overlaps a destination");
+  a.src = src;
+  a.src_pstride = src_pstride;
+  a.blocked = 1;
+  hipError_t e = launch_ntt_fwd_rows(a, num_limbs, num_polys, kEpiModDown,
+                                     static_cast<hipStream_t>(stream));
+  if (e != hipSuccess)
+    return set_error(CHD_ERR_HIP,
+                     std::string(who) + ": " + hipGetErrorString(e));
+  return 0;
+}
+
 extern "C" int chd_k_ntt_fwd_moddown_multi(
     const chd_tables *t, const chd_limb_map *m, uint32_t *const *dst,
     int num_polys, int num_limbs, const uint32_t *src, long long src_pstride,
@@ -2306,12 +2493,7 @@ extern "C" int chd_k_ntt_fwd_moddown_multi(
     return st;
   if (src != nullptr) {
     // separate source: single-pass kernel when no destination overlaps it
-    bool ok = true;
-    for (int p = 0; p < num_polys; p++)
-      ok = ok && sets_disjoint(src, src_pstride, num_polys,
-                               span_limbs(num_limbs, a.map, true), dst[p], 0,
-                               1, span_limbs(num_limbs, a.map, false));
-    if (!ok)
+    if (!moddown_src_disjoint(a, src, src_pstride, num_polys, num_limbs))
       return set_error(CHD_ERR_ARG,
                        "chd_k_ntt_fwd_moddown_multi: source overlaps a "
                        "destination");

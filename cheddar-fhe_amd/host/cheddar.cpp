@@ -25,23 +25,6 @@ void K(int status) {
 
 int DivCeil(int a, int b) { return (a + b - 1) / b; }
 
-// ModDown's destination-limb counts (polynomials x limbs) up to which the
-// BConv writes the destination and a two-pass NTT runs in place on it; above
-// them a single-pass NTT does. The one-source case (Rescale) has its own,
-// lower limit: there the single pass forms the BConv itself and saves a
-// launch. Measured on MI355X, warm, microseconds (threshold 32 / single pass
-// everywhere / two passes everywhere):
-//   ModDown, 1 poly, 8..24 limbs: 28.2..33.2 / 32.4..37.8 / 28.2..33.2
-//   HMult (merged rescale), 2 x 19 and 2 x 23 limbs: 86.9, 89.0 / 86.8,
-//     88.9 / 88.1, 91.2; 2 x 15: 70.4 (two passes) / 70.9 (single)
-//   Rescale, 1 poly, 7 / 11 / 15 / 19 / 23 limbs: two passes 25.8 / 27.0 /
-//     28.2 / 30.5 / 31.3, single pass 27.6 / 27.5 / 27.7 / 28.1 / 27.8
-#ifndef CHD_SMALL_MODDOWN_LIMBS
-#define CHD_SMALL_MODDOWN_LIMBS 32
-#endif
-#ifndef CHD_SMALL_RESCALE_LIMBS
-#define CHD_SMALL_RESCALE_LIMBS 12
-#endif
 // 1: a hoisting handle with a wide giant-step accumulation keeps a tiled
 // copy of its plaintexts beside the per-pair ones (twice their memory); 0:
 // the accumulation reads the per-pair plaintexts in place
@@ -836,121 +819,71 @@ void ModSwitchHandler<uint32_t>::BuildSwitch(
   K(chd_bconv_table_pack(packed.data(), c2.data(), dst.data(), sl, dl));
   st.table.Resize(packed.size());
   st.table.Upload(packed.data(), packed.size());
-  if (sl == 1) {
-    std::vector<word> col(dl);
-    for (int k = 0; k < dl; k++)
-      col[k] = c2[k] < 0 ? static_cast<word>(c2[k] + static_cast<int64_t>(dst[k]))
-                         : static_cast<word>(c2[k]);
-    st.bconv1.resize(dl);
-    HipCheck(hipMemcpy(st.bconv1.data(), col.data(), dl * sizeof(word),
-                       hipMemcpyHostToDevice),
-             "hipMemcpy");
-  }
 }
 
-// src/core/ModSwitch.cu:429-485: INTTAndMultConst(centre) of src into intt,
-// then the BConv of every dnum group in one launch, group i into dst[i].
-void ModSwitchHandler<uint32_t>::ModUpBconv(word *const *dst,
-                                            const DvConstView<word> &src,
-                                            word *intt,
-                                            const word *src_mul) const {
-  const NPInfo np = param_.LevelToNP(level_, 0);
-  const int num_q = np.GetNumQ();
-  const int n = param_.degree_;
-  AssertTrue(src.QSize() == num_q * n, "ModUp src q size mismatch");
-  AssertTrue(src.AuxSize() == 0, "ModUp src aux size mismatch");
-  AssertTrue(NumGroups() <= CHD_MAX_JOBS, "ModUp: dnum larger than supported");
-  if (src_mul != nullptr) {
-    const chd_limb_map mi = NoSkipMap(param_, np);
-    K(chd_k_ntt_inv_mul(&ntt_.Tables(), &mi, intt, 0, src.data(), src_mul, 0,
-                        num_q, 1, mod_up1_.data(), 1, CurrentStream()));
-  } else {
-    DvView<word> intt_view(intt, num_q * n, 0);
-    ntt_.INTTAndMultConst(intt_view, np, src,
-                          DvConstView<word>(mod_up1_.data(), num_q, 0), true);
-  }
-  NPInfo np_aux = np;
-  np_aux.num_aux_ = num_aux_;
-  chd_limb_map m = NoSkipMap(param_, np_aux);
-  chd_bconv_job jobs[CHD_MAX_JOBS] = {};
-  for (int z = 0; z < NumGroups(); z++) {
-    const int s0 = GroupLo(z), s1 = GroupHi(z);
-    const SwitchTable &st = mod_up_[z];
-    jobs[z].dst = dst[z];
-    jobs[z].src = reinterpret_cast<const int32_t *>(intt) +
-                  static_cast<size_t>(s0) * n;
-    jobs[z].table = st.table.as<void>();
-    jobs[z].src_len = st.src_len;
-    jobs[z].dst_len = st.dst_len;
-    jobs[z].skip_lo = s0;
-    jobs[z].skip_len = s1 - s0;
-  }
-  K(chd_k_bconv_batch(&ntt_.Tables(), &m, jobs, NumGroups(), CurrentStream()));
-}
-
-// ModUp with every group's column pass (and, with_rows, row pass) batched;
-// group i lives at modup + i * group_stride. Own limbs are not written.
-void ModSwitchHandler<uint32_t>::ModUpGroups(word *modup,
-                                             long long group_stride,
-                                             const DvConstView<word> &src,
-                                             word *intt, bool with_rows,
-                                             const word *src_mul) const {
-  const NPInfo np = param_.LevelToNP(level_, 0);
-  const int num_q = np.GetNumQ();
-  word *dst[CHD_MAX_JOBS];
-  AssertTrue(NumGroups() <= CHD_MAX_JOBS, "ModUp: dnum larger than supported");
-  for (int z = 0; z < NumGroups(); z++) dst[z] = modup + z * group_stride;
-  ModUpBconv(dst, src, intt, src_mul);
-  NPInfo np_aux = np;
-  np_aux.num_aux_ = num_aux_;
-  chd_limb_map m = NoSkipMap(param_, np_aux);
-  K(chd_k_ntt_fwd_groups(&ntt_.Tables(), &m, modup, group_stride, NumGroups(),
-                         num_aux_, group_shift_, num_q + num_aux_,
-                         with_rows ? 1 : 0, CurrentStream()));
-}
-
-void ModSwitchHandler<uint32_t>::ModUpGroupsBatch(word *modup,
-                                                  long long group_stride,
-                                                  const word *src,
-                                                  long long src_stride,
-                                                  int num_inputs,
-                                                  word *intt) const {
+// src/core/ModSwitch.cu:429-509 up to the forward row pass: the inverse row
+// pass of every input into intt, then the column stage of every input's dnum
+// groups in one launch. Own limbs are not written.
+void ModSwitchHandler<uint32_t>::ModUpColumns(word *modup,
+                                              long long group_stride,
+                                              const word *src,
+                                              long long src_stride,
+                                              int num_inputs, word *intt,
+                                              const word *src_mul) const {
   const NPInfo np = param_.LevelToNP(level_, 0);
   const int num_q = np.GetNumQ();
   const int n = param_.degree_;
   const int groups = NumGroups();
+  AssertTrue(groups <= CHD_MAX_JOBS, "ModUp: dnum larger than supported");
   AssertTrue(num_inputs >= 1 && num_inputs <= CHD_MAX_JOBS,
              "ModUp: 1 to CHD_MAX_JOBS inputs per batch");
   AssertTrue(groups * num_inputs <= CHD_MAX_BCONV_JOBS,
              "ModUp: too many groups in one batch");
-  // INTTAndMultConst(centre) of every input (ModSwitch.cu:442-447)
   const chd_limb_map mi = NoSkipMap(param_, np);
   const long long ilen = static_cast<long long>(num_q) * n;
-  K(chd_k_ntt_inv(&ntt_.Tables(), &mi, intt, ilen, src, src_stride, num_q,
-                  num_inputs, mod_up1_.data(), 1, CurrentStream()));
+  K(chd_k_ntt_inv_rows(&ntt_.Tables(), &mi, intt, ilen, src, src_mul,
+                       src_stride, num_q, num_inputs, CurrentStream()));
   NPInfo np_aux = np;
   np_aux.num_aux_ = num_aux_;
-  chd_limb_map m = NoSkipMap(param_, np_aux);
-  chd_bconv_job jobs[CHD_MAX_BCONV_JOBS] = {};
+  const chd_limb_map m = NoSkipMap(param_, np_aux);
+  chd_switch_job jobs[CHD_MAX_BCONV_JOBS] = {};
   for (int i = 0; i < num_inputs; i++)
     for (int z = 0; z < groups; z++) {
       const int s0 = GroupLo(z), s1 = GroupHi(z);
       const SwitchTable &st = mod_up_[z];
-      chd_bconv_job &jb = jobs[i * groups + z];
+      chd_switch_job &jb = jobs[i * groups + z];
       jb.dst = modup + (static_cast<long long>(i) * groups + z) * group_stride;
-      jb.src = reinterpret_cast<const int32_t *>(intt) + i * ilen +
-               static_cast<size_t>(s0) * n;
+      jb.src = intt + i * ilen + static_cast<size_t>(s0) * n;
+      jb.src_cst = mod_up1_.data() + s0;
       jb.table = st.table.as<void>();
       jb.src_len = st.src_len;
       jb.dst_len = st.dst_len;
       jb.skip_lo = s0;
       jb.skip_len = s1 - s0;
+      jb.src_tab = mi.tab_off + s0;
+      jb.src_num_q = st.src_len;
     }
-  K(chd_k_bconv_batch(&ntt_.Tables(), &m, jobs, groups * num_inputs,
+  K(chd_k_switch_cols(&ntt_.Tables(), &m, jobs, groups * num_inputs,
                       CurrentStream()));
-  K(chd_k_ntt_fwd_groups_batch(&ntt_.Tables(), &m, modup, group_stride,
-                               groups, num_inputs, num_aux_, group_shift_,
-                               num_q + num_aux_, 0, CurrentStream()));
+}
+
+size_t ModSwitchHandler<uint32_t>::ModUpScratchWords() const {
+  const size_t num_q = param_.LevelToNP(level_).GetNumQ();
+  return (num_q + NumGroups() * (num_q + num_aux_)) * param_.degree_;
+}
+
+void ModSwitchHandler<uint32_t>::ModUpGroups(word *const *dst, const word *src,
+                                             word *scratch) const {
+  NPInfo np = param_.LevelToNP(level_, num_aux_);
+  const int num_q = np.GetNumQ();
+  const long long gs =
+      static_cast<long long>(num_q + num_aux_) * param_.degree_;
+  word *const blocked = scratch + static_cast<size_t>(num_q) * param_.degree_;
+  ModUpColumns(blocked, gs, src, 0, 1, scratch);
+  const chd_limb_map m = NoSkipMap(param_, np);
+  K(chd_k_ntt_fwd_rows_groups(&ntt_.Tables(), &m, dst, blocked, gs,
+                              NumGroups(), num_aux_, group_shift_,
+                              num_q + num_aux_, CurrentStream()));
 }
 
 // src/core/ModSwitch.cu:429-509
@@ -961,14 +894,15 @@ void ModSwitchHandler<uint32_t>::ModUp(std::vector<DvView<word>> &dst,
   const int n = param_.degree_;
   AssertTrue(static_cast<int>(dst.size()) == beta_, "ModUp dst size mismatch");
   AssertTrue(NumGroups() <= CHD_MAX_JOBS, "ModUp: dnum larger than supported");
-  const long long gs = static_cast<long long>(num_q + num_aux_) * n;
+  AssertTrue(src.QSize() == num_q * n, "ModUp src q size mismatch");
+  AssertTrue(src.AuxSize() == 0, "ModUp src aux size mismatch");
   const int first = first_group_;
-  bool strided = true;
+  word *d[CHD_MAX_JOBS];
   for (int z = 0; z < NumGroups(); z++) {
-    const DvView<word> &d = dst[first + z];
-    AssertTrue(d.AuxSize() == num_aux_ * n && d.QSize() == num_q * n,
+    const DvView<word> &v = dst[first + z];
+    AssertTrue(v.AuxSize() == num_aux_ * n && v.QSize() == num_q * n,
                "ModUp dst size mismatch");
-    strided = strided && d.data() == dst[first].data() + z * gs;
+    d[z] = dst[first + z].data();
   }
   // own limbs are the input's (ModSwitch.cu:449-470); groups before
   // FirstGroup() hold no limb of this level and are not written
@@ -981,19 +915,8 @@ void ModSwitchHandler<uint32_t>::ModUp(std::vector<DvView<word>> &dst,
              "hipMemcpyAsync");
   }
   Workspace::Use use_ws(ws_);
-  Scratch intt(ws_, static_cast<size_t>(num_q) * n);
-  if (strided) {  // groups equally spaced: one launch per pass for all
-    ModUpGroups(dst[first].data(), gs, src, intt.data(), true);
-    return;
-  }
-  word *d[CHD_MAX_JOBS];
-  for (int z = 0; z < NumGroups(); z++) d[z] = dst[first + z].data();
-  ModUpBconv(d, src, intt.data());
-  NPInfo np_aux = np;
-  np_aux.num_aux_ = num_aux_;
-  for (int z = 0; z < NumGroups(); z++)
-    ntt_.NTTForModUp(dst[first + z], np_aux, GroupLo(z), GroupHi(z),
-                     DvConstView<word>(dst[first + z]));
+  Scratch tmp(ws_, ModUpScratchWords());
+  ModUpGroups(d, src.data(), tmp.data());
 }
 
 // src/core/ModSwitch.cu:414-428 (MultConst by p_prod)
@@ -1168,15 +1091,12 @@ void ModSwitchHandler<uint32_t>::ModDownMulti(const std::vector<word *> &dst,
     mi.tab_gap = param_.GetMaxNumMain() + np_non_intt.num_ter_;
     mi.src_gap = np_src.GetNumQ() - mi.num_q;
   }
-  if (intt_rows != nullptr) {
+  if (intt_rows != nullptr)
     // the first pass was done by the key accumulation (ModDownInttRange)
     AssertTrue(!intt_on_ter, "ModDown: fused INTT needs main INTT limbs");
-    K(chd_k_ntt_inv_cols(&ntt_.Tables(), &mi, intt, ilen, src_len, num_polys,
-                         st.const1.data(), 1, CurrentStream()));
-  } else {
-    K(chd_k_ntt_inv(&ntt_.Tables(), &mi, intt, ilen, src + off, src_pstride,
-                    src_len, num_polys, st.const1.data(), 1, CurrentStream()));
-  }
+  else
+    K(chd_k_ntt_inv_rows(&ntt_.Tables(), &mi, intt, ilen, src + off, nullptr,
+                         src_pstride, src_len, num_polys, CurrentStream()));
   chd_limb_map m = NoSkipMap(param_, np_dst);
   const DeviceVector<word> &ipp =
       kind == Kind::ModDown   ? inv_prime_prod_
@@ -1190,58 +1110,31 @@ void ModSwitchHandler<uint32_t>::ModDownMulti(const std::vector<word *> &dst,
                                        : mod_down_rescale_padding_;
   const word *pad =
       kind != Kind::ModDown && padv.size() != 0 ? padv.data() : nullptr;
-  // NTTForModDown (NTT.cu:417-604) with src2 = the untouched low limbs
-  // (src2_off, s2_lo, s2_hi above). Few destination limbs: the single-pass NTT's time is one workgroup's
-  // latency (~15 us whatever the limb count), so the BConv writes the
-  // destination and the two-pass NTT runs in place on it, its passes
-  // spread over many small workgroups (HMult at L = 4, 8, 12, 16: 6.4, 5.8,
-  // 3.2 and 2.2 us faster; at 38 and 46 limbs the single pass is ahead)
-  const bool one_src =
-      st.src_len == 1 && st.bconv1.size() == static_cast<size_t>(dst_len);
-  const bool few = num_polys * dst_len <= (one_src ? CHD_SMALL_RESCALE_LIMBS
-                                                   : CHD_SMALL_MODDOWN_LIMBS);
-  if (!few && one_src) {
-    // one source (Rescale): the NTT forms each limb's BConv, the source
-    // times that limb's table entry, from the one INTT limb as it reads it
-    K(chd_k_ntt_fwd_moddown_bconv1_multi(
-        &ntt_.Tables(), &m, dst.data(), num_polys, dst_len,
-        reinterpret_cast<const int32_t *>(intt), ilen, st.bconv1.data(),
-        src + static_cast<size_t>(src2_off) * n, src_pstride, s2_lo, s2_hi,
-        ipp.data(), pad, CurrentStream()));
-    return;
-  }
-  chd_bconv_job jobs[CHD_MAX_JOBS] = {};
-  for (int p = 0; p < num_polys; p++) {
-    jobs[p].dst = dst[p];
-    jobs[p].src = reinterpret_cast<const int32_t *>(intt) + p * ilen;
-    jobs[p].table = st.table.as<void>();
-    jobs[p].src_len = src_len;
-    jobs[p].dst_len = dst_len;
-    jobs[p].skip_lo = INT_MAX;
-    jobs[p].skip_len = 0;
-  }
-  if (few) {
-    K(chd_k_bconv_batch(&ntt_.Tables(), &m, jobs, num_polys,
-                        CurrentStream()));
-    K(chd_k_ntt_fwd_moddown_multi(&ntt_.Tables(), &m, dst.data(), num_polys,
-                                  dst_len, nullptr, 0,
-                                  src + static_cast<size_t>(src2_off) * n,
-                                  src_pstride, s2_lo, s2_hi, ipp.data(), pad,
-                                  CurrentStream()));
-    return;
-  }
-  // BConv into a temporary so that the NTT below reads it and writes dst in
-  // one pass (the single-pass forward NTT cannot run in place)
+  // the column stage, then the row pass with the epilogue (NTTForModDown,
+  // NTT.cu:417-604) whose src2 are the untouched low limbs (src2_off, s2_lo,
+  // s2_hi above)
   Scratch conv(ws_, static_cast<size_t>(num_polys) * dst_len * n);
-  for (int p = 0; p < num_polys; p++)
-    jobs[p].dst = conv.data() + static_cast<size_t>(p) * dst_len * n;
-  K(chd_k_bconv_batch(&ntt_.Tables(), &m, jobs, num_polys, CurrentStream()));
-  K(chd_k_ntt_fwd_moddown_multi(&ntt_.Tables(), &m, dst.data(), num_polys,
-                                dst_len, conv.data(),
-                                static_cast<long long>(dst_len) * n,
-                                src + static_cast<size_t>(src2_off) * n,
-                                src_pstride, s2_lo, s2_hi, ipp.data(), pad,
-                                CurrentStream()));
+  const long long clen = static_cast<long long>(dst_len) * n;
+  chd_switch_job jobs[CHD_MAX_JOBS] = {};
+  for (int p = 0; p < num_polys; p++) {
+    chd_switch_job &jb = jobs[p];
+    jb.dst = conv.data() + p * clen;
+    jb.src = intt + p * ilen;
+    jb.src_cst = st.const1.data();
+    jb.table = st.table.as<void>();
+    jb.src_len = src_len;
+    jb.dst_len = dst_len;
+    jb.skip_lo = INT_MAX;
+    jb.src_tab = mi.tab_off;
+    jb.src_num_q = mi.num_q;
+    jb.src_tab_gap = mi.tab_gap;
+  }
+  K(chd_k_switch_cols(&ntt_.Tables(), &m, jobs, num_polys, CurrentStream()));
+  K(chd_k_ntt_fwd_rows_moddown(&ntt_.Tables(), &m, dst.data(), num_polys,
+                               dst_len, conv.data(), clen,
+                               src + static_cast<size_t>(src2_off) * n,
+                               src_pstride, s2_lo, s2_hi, ipp.data(), pad,
+                               CurrentStream()));
 }
 
 // ---------------------------------------------------------------- Context --
@@ -1530,9 +1423,8 @@ void Context<uint32_t>::KeyAccumulate(int level, word *acc_b, word *acc_a,
   Scratch buf(ws_.get(),
               static_cast<size_t>(groups) * gs + static_cast<size_t>(num_q) * n);
   const bool tensor = ta != nullptr;
-  ms.ModUpGroups(buf.data(), gs,
-                 DvConstView<word>(tensor ? ta->ax : d, num_q * n, 0),
-                 buf.data() + groups * gs, false, tensor ? tb->ax : nullptr);
+  ms.ModUpColumns(buf.data(), gs, tensor ? ta->ax : d, 0, 1,
+                  buf.data() + groups * gs, tensor ? tb->ax : nullptr);
   chd_keyacc_args k{};
   k.num_q = num_q;
   k.tab_off = param_.TerLeft(a_np);
@@ -1542,6 +1434,7 @@ void Context<uint32_t>::KeyAccumulate(int level, word *acc_b, word *acc_a,
   k.group_shift = ms.GroupShift();
   k.modup = buf.data();
   k.group_stride = gs;
+  k.blocked = 1;
   k.d = d;
   for (int z = 0; z < groups; z++) {
     k.kb[z] = key.bx[first + z] + static_cast<size_t>(prime_offset) * n;
@@ -1596,8 +1489,8 @@ void Context<uint32_t>::KeyMultExtBatchV(int level, int num,
   Workspace::Use use_ws(ws_.get());
   Scratch buf(ws_.get(), static_cast<size_t>(num) * groups * gs +
                              static_cast<size_t>(num) * num_q * n);
-  ms.ModUpGroupsBatch(buf.data(), gs, d, d_stride, num,
-                      buf.data() + static_cast<size_t>(num) * groups * gs);
+  ms.ModUpColumns(buf.data(), gs, d, d_stride, num,
+                  buf.data() + static_cast<size_t>(num) * groups * gs);
   chd_keyacc_args jobs[CHD_MAX_JOBS] = {};
   for (int i = 0; i < num; i++) {
     const EvkRef &key = *keys[i];
@@ -1615,6 +1508,7 @@ void Context<uint32_t>::KeyMultExtBatchV(int level, int num,
     k.group_shift = ms.GroupShift();
     k.modup = buf.data() + static_cast<size_t>(i) * groups * gs;
     k.group_stride = gs;
+    k.blocked = 1;
     k.d = d + i * d_stride;
     for (int z = 0; z < groups; z++) {
       k.kb[z] = key.bx[first + z] + static_cast<size_t>(prime_offset) * n;
@@ -2294,12 +2188,13 @@ void HoistHandler<uint32_t>::BabyStep(const Context<word> &ctx,
     if (b != 0) rots.push_back(b);
   // 1. ModUp of a, all groups (own limbs are read from a by the kernel)
   const long long gs = static_cast<long long>(total) * n;
-  Scratch buf(ws, rots.empty() ? 0
-                               : static_cast<size_t>(beta) * gs +
-                                     static_cast<size_t>(num_q) * n);
-  if (!rots.empty())
-    ms.ModUpGroups(buf.data(), gs, input.ax_.ConstView(),
-                   buf.data() + beta * gs, true);
+  Scratch buf(ws, rots.empty() ? 0 : static_cast<size_t>(beta) * gs);
+  if (!rots.empty()) {
+    Scratch tmp(ws, ms.ModUpScratchWords());
+    word *d[CHD_MAX_BS_GROUPS];
+    for (int g = 0; g < beta; g++) d[g] = buf.data() + g * gs;
+    ms.ModUpGroups(d, input.ax_.data(), tmp.data());
+  }
   // 2. baby step 0: the PseudoModUp of (b, a), zero on the aux limbs
   auto slot = [&](int idx) -> Ct & {
     Ct &ct = bs.try_emplace(idx, ext_np).first->second;

@@ -610,27 +610,22 @@ class ModSwitchHandler<uint32_t> {
   void PseudoModUp(DvView<word> &dst, const DvConstView<word> &src,
                    const DvConstView<word> &p_prod) const;
 
-  // Batched pieces of ModUp used by the fused key switch (no single
-  // reference counterpart). ModUpBconv: INTTAndMultConst(centre) of src into
-  // intt (num_q limbs) and the BConv of every dnum group i into dst[i].
-  // ModUpGroups: ModUpBconv into modup + i * group_stride, then the column
-  // pass (with_rows: and the row pass) of NTTForModUp for all groups in one
-  // launch each. Own limbs of a group are left unwritten.
-  // With src_mul, the ModUp input is the element-wise MontMul(src, src_mul)
-  // (the Tensor's rx of HMult, formed on the fly).
-  void ModUpBconv(word *const *dst, const DvConstView<word> &src,
-                  word *intt, const word *src_mul = nullptr) const;
-  void ModUpGroups(word *modup, long long group_stride,
-                   const DvConstView<word> &src, word *intt,
-                   bool with_rows, const word *src_mul = nullptr) const;
-  // ModUpGroups (column passes only) of num_inputs (<= CHD_MAX_JOBS)
-  // independent inputs of this level in one launch per phase: input i is
-  // src + i * src_stride (num_q limbs), its group z goes to
-  // modup + (i * NumGroups() + z) * group_stride, and intt holds
-  // num_inputs * num_q limbs of scratch.
-  void ModUpGroupsBatch(word *modup, long long group_stride, const word *src,
-                        long long src_stride, int num_inputs,
-                        word *intt) const;
+  // Pieces of ModUp used by the fused key switch (no single reference
+  // counterpart). ModUpColumns: everything up to the forward row pass for
+  // num_inputs (<= CHD_MAX_JOBS) independent inputs of this level, one launch
+  // per phase: input i is src + i * src_stride (num_q limbs), its group z
+  // goes, column-blocked (cheddar_kernels.h), to
+  // modup + (i * NumGroups() + z) * group_stride; intt holds
+  // num_inputs * num_q limbs of scratch. With src_mul, the input is the
+  // element-wise MontMul(src, src_mul) (the Tensor's rx of HMult, formed on
+  // the fly). ModUpGroups: the whole ModUp of one input, group z into dst[z]
+  // (num_q + alpha limbs in the usual order), with ModUpScratchWords() words
+  // of scratch. Own limbs of a group are left unwritten.
+  void ModUpColumns(word *modup, long long group_stride, const word *src,
+                    long long src_stride, int num_inputs, word *intt,
+                    const word *src_mul = nullptr) const;
+  void ModUpGroups(word *const *dst, const word *src, word *scratch) const;
+  size_t ModUpScratchWords() const;
 
   enum class Kind { ModDown, Rescale, ModDownAndRescale };
   // ModDownWorker for several polynomials at once: polynomial p of the
@@ -638,8 +633,8 @@ class ModSwitchHandler<uint32_t> {
   // polynomials may sit in separate allocations), its result goes to
   // dst[p] (separate buffers allowed).
   // intt_rows: when given, the first pass of the INTT (stages 15..8) of the
-  // INTT limbs is already there ([polynomial][limb] of the INTT limbs, as
-  // the key accumulation leaves it), and only the second pass runs.
+  // INTT limbs is already there ([polynomial][limb] of the INTT limbs,
+  // column-blocked, as the key accumulation leaves it).
   void ModDownMulti(const std::vector<word *> &dst, const word *src,
                     long long src_pstride, Kind kind,
                     word *intt_rows = nullptr) const;
@@ -657,9 +652,6 @@ class ModSwitchHandler<uint32_t> {
   struct SwitchTable {       // one source set -> destination set
     DeviceVector<word> const1;   // (N prod_{j!=i} s_j)^-1 mod s_i
     DevBuf table;                // packed BConv table (chd_bconv_table_pack)
-    // one source only: its table column, canonical per destination (the
-    // NTT of the ModDown tail then forms the BConv itself)
-    DeviceVector<word> bconv1;
     int src_len = 0, dst_len = 0;
   };
   // restore: destination primes [restore_lo, restore_hi) come back without

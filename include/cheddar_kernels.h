@@ -173,6 +173,54 @@ typedef struct chd_bconv_job {
 int chd_k_bconv_batch(const chd_tables *t, const chd_limb_map *m,
                       const chd_bconv_job *jobs, int num_jobs, void *stream);
 
+/* A base switch (ModUp, ModDown, Rescale) as three launches: the inverse row
+ * pass, the column stage, the forward row pass. Between them limbs are
+ * column-blocked: index row * 256 + col of a limb sits at word
+ * ((col >> 2) * 256 + row) * 4 + (col & 3), unreduced.
+ *
+ * chd_k_ntt_inv_rows: the first pass (stages 15..8) of chd_k_ntt_inv, or of
+ * chd_k_ntt_inv_mul when src_mul is given, into column-blocked dst, which
+ * must not overlap a source. */
+int chd_k_ntt_inv_rows(const chd_tables *t, const chd_limb_map *m,
+                       uint32_t *dst, long long dst_pstride,
+                       const uint32_t *src, const uint32_t *src_mul,
+                       long long src_pstride, int num_limbs, int num_polys,
+                       void *stream);
+/* The column stage of up to CHD_MAX_BCONV_JOBS switches in one launch: the
+ * second pass of the inverse NTT with its centred constant, the BConv and
+ * the first pass of the forward NTT (ModSwitch.cu:429-684 without the row
+ * passes). Source i of a job is src + i N, its prime
+ * src_tab + i + (i >= src_num_q ? src_tab_gap : 0), its constant src_cst[i];
+ * destination k goes to limb pos(k) of dst as in chd_bconv_job, its prime
+ * through m. dst must not overlap a source; 1 <= src_len <= 32. */
+typedef struct chd_switch_job {
+  uint32_t *dst;
+  const uint32_t *src;
+  const uint32_t *src_cst;
+  const void *table; /* chd_bconv_table_pack(src_len, dst_len) */
+  int src_len, dst_len;
+  int skip_lo, skip_len;
+  int src_tab, src_num_q, src_tab_gap;
+} chd_switch_job;
+int chd_k_switch_cols(const chd_tables *t, const chd_limb_map *m,
+                      const chd_switch_job *jobs, int num_jobs, void *stream);
+/* The second pass (stages 8..15) of chd_k_ntt_fwd_moddown_multi on
+ * column-blocked input src + p * src_pstride; no dst[p] may overlap it. */
+int chd_k_ntt_fwd_rows_moddown(const chd_tables *t, const chd_limb_map *m,
+                               uint32_t *const *dst, int num_polys,
+                               int num_limbs, const uint32_t *src,
+                               long long src_pstride, const uint32_t *src2,
+                               long long src2_pstride, int src2_lo,
+                               int src2_hi, const uint32_t *inv_prod,
+                               const uint32_t *pad, void *stream);
+/* The second pass of chd_k_ntt_fwd_groups (num_groups <= CHD_MAX_JOBS) from
+ * column-blocked src + g * group_stride into dst[g], own limbs skipped. */
+int chd_k_ntt_fwd_rows_groups(const chd_tables *t, const chd_limb_map *m,
+                              uint32_t *const *dst, const uint32_t *src,
+                              long long group_stride, int num_groups,
+                              int alpha, int group_shift, int group_limbs,
+                              void *stream);
+
 /* Column pass (stages 0..7) of NTTForModUp for all dnum groups in one launch:
  * group g's polynomial sits at modup + g * group_stride (group_limbs limbs,
  * in place) and its own limbs [max(0, g alpha - group_shift),
@@ -233,6 +281,9 @@ typedef struct chd_keyacc_args {
    * intt_{b,a} + (l - intt_lo) N instead, for chd_k_ntt_inv_cols to finish */
   uint32_t *intt_b, *intt_a;
   int intt_lo;
+  /* non-zero: modup is column-blocked (chd_k_switch_cols), and so is what
+   * goes to intt_{b,a} */
+  int blocked;
 } chd_keyacc_args;
 int chd_k_modup_keyacc(const chd_tables *t, const chd_keyacc_args *args,
                        void *stream);
