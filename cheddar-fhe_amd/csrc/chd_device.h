@@ -118,6 +118,15 @@ inline bool groups_valid(int beta, int alpha, int shift, int num_q) {
          (beta - 1) * alpha - shift < num_q && beta * alpha - shift >= num_q;
 }
 
+// index map of the NTT-domain automorphism (ElementWise.cu:370-391):
+// dst[x] = src[perm_index(x, galois)]. The top k bits of the result depend
+// on the top k bits of x alone (they are the low bits of 2 brev(x) + 1, which
+// an odd factor maps among themselves), so rows of 256 map to whole rows.
+__device__ __forceinline__ uint32_t perm_index(uint32_t x, uint32_t galois) {
+  const uint32_t e = (__brev(x) >> (32 - (kLogN + 1))) + 1;
+  return __brev(e * galois - 1) >> (32 - (kLogN + 1));
+}
+
 // wave-uniform value into an SGPR
 __device__ __forceinline__ int uniform(int v) {
   return __builtin_amdgcn_readfirstlane(v);

@@ -184,23 +184,13 @@ __global__ __launch_bounds__(kThreads) void permute_kernel(chd_limb_map m,
   const int c0 = blockIdx.x * kCoefPerBlock + threadIdx.x * kPerThread;
   uint32_t idx[4];
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    uint32_t x = c0 + i;
-    uint32_t e = (__brev(x) >> (32 - (kLogN + 1))) + 1;
-    idx[i] = __brev(e * galois - 1) >> (32 - (kLogN + 1));
-  }
+  for (int i = 0; i < 4; i++) idx[i] = perm_index(c0 + i, galois);
 #pragma unroll
   for (int p = 0; p < kPoly; p++) {
     const uint32_t *s = a.src[p] + sbase;
     st4(a.dst[p] + base + c0,
         make_uint4(s[idx[0]], s[idx[1]], s[idx[2]], s[idx[3]]));
   }
-}
-
-// galois index map of Permute (ElementWise.cu:370-391): dst[x] = src[perm(x)]
-__device__ __forceinline__ uint32_t perm_index(uint32_t x, uint32_t galois) {
-  const uint32_t e = (__brev(x) >> (32 - (kLogN + 1))) + 1;
-  return __brev(e * galois - 1) >> (32 - (kLogN + 1));
 }
 
 __global__ __launch_bounds__(kThreads) void zero_kernel(uint4 *dst,

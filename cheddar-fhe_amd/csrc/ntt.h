@@ -16,6 +16,7 @@ enum NttEpilogue : int {
   kEpiModDown = 1,   // MontMul(MontMul(src2,pad) - y, cst2)
   kEpiConst = 2,     // MontMul(y, cst)
   kEpiConstCentre = 3,
+  kEpiModDownPerm = 4,  // kEpiModDown, then the automorphism galois
 };
 
 struct NttArgs {
@@ -63,6 +64,8 @@ struct NttArgs {
   // row passes only: the input (forward) or output (inverse) is
   // column-blocked and apart from the other side
   int blocked;
+  // kEpiModDownPerm only: the automorphism's factor and its inverse mod 2N
+  uint32_t galois, galois_inv;
 };
 
 // Fused ModUp row pass + evaluation-key inner product (PAccum) + CAccum for

@@ -580,14 +580,15 @@ __device__ __forceinline__ void fwd_rows_body(const NttArgs &a, const Limb &lb,
   char *tile = reinterpret_cast<char *>(dst) + tile_byte(kBlocked);
   [[maybe_unused]] const int32_t qs = static_cast<int32_t>(q);
   [[maybe_unused]] int32_t c2 = 0, c2q = 0;
-  if constexpr (kEpi == kEpiModDown) {
+  constexpr bool kDown = kEpi == kEpiModDown || kEpi == kEpiModDownPerm;
+  if constexpr (kDown) {
     c2 = static_cast<int32_t>(a.cst2[lb.l]);
     c2q = static_cast<int32_t>(static_cast<uint32_t>(c2) * qinv);
   }
 #pragma unroll
   for (int v = 0; v < 4; v++) {
     u32x4 o = tile_lds4(xt, v);
-    if constexpr (kEpi == kEpiModDown) {
+    if constexpr (kDown) {
       // NTTPhase2ForModDown epilogue (NTT.cu:567-600); src2 (and its
       // optional padding product) was loaded before the butterflies
 #pragma unroll
@@ -597,7 +598,27 @@ __device__ __forceinline__ void fwd_rows_body(const NttArgs &a, const Limb &lb,
         o[j] = static_cast<uint32_t>(norm(mont(d, c2, c2q, qs), qs));
       }
     }
-    st_nt<u32x4>(tile, tile_lane_byte(kBlocked, v), o);
+    if constexpr (kEpi == kEpiModDownPerm) {
+      // the automorphism maps this wave's row to a whole row: its columns
+      // are reordered through the row's own LDS words, and it is stored as
+      // that row (1 KiB per wave as before), where a permutation of its own
+      // would read and write every limb once more
+      const int rr = static_cast<int>(threadIdx.x >> 6) + 4 * v;
+      const int lane = threadIdx.x & 63;
+      uint32_t *row = reinterpret_cast<uint32_t *>(xch) + rr * kRowPad;
+#pragma unroll
+      for (int j = 0; j < 4; j++) row[pidx(4 * lane + j)] = o[j];
+      wave_lds_sync();
+      const uint32_t to =
+          perm_index(static_cast<uint32_t>(tile_row(kBlocked, rr)) << 8,
+                     a.galois_inv) >> 8;
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        o[j] = row[pidx(perm_index((to << 8) + 4 * lane + j, a.galois) & 255)];
+      st_nt<u32x4>(dst, to * (kCols * 4u) + 16u * lane, o);
+    } else {
+      st_nt<u32x4>(tile, tile_lane_byte(kBlocked, v), o);
+    }
   }
 }
 
@@ -637,7 +658,8 @@ __global__ __launch_bounds__(256) void ntt_fwd_rows(NttArgs a) {
   // coalesced store layout (zero outside [src2_lo, src2_hi)), loaded with the
   // data so their latency hides behind the butterflies
   uint32_t s2v[16] = {};
-  if constexpr (kEpi == kEpiModDown) {
+  constexpr bool kDown = kEpi == kEpiModDown || kEpi == kEpiModDownPerm;
+  if constexpr (kDown) {
     if (lb.l >= a.src2_lo && lb.l < a.src2_hi) {
       const uint32_t *s2p = a.src2 + blockIdx.z * a.src2_pstride +
                             (static_cast<size_t>(lb.l - a.src2_lo) << kLogN);
@@ -655,7 +677,7 @@ __global__ __launch_bounds__(256) void ntt_fwd_rows(NttArgs a) {
   }
   const uint32_t q = a.tab.q[lb.ti];
   const uint32_t qinv = static_cast<uint32_t>(a.tab.qinv[lb.ti]);
-  if constexpr (kEpi == kEpiModDown) {
+  if constexpr (kDown) {
     if (a.pad != nullptr && lb.l >= a.src2_lo && lb.l < a.src2_hi) {
       // src2 * padding (BitPacker restore, NTT.cu:579-585)
       const int32_t qs = static_cast<int32_t>(q);
@@ -1893,7 +1915,9 @@ hipError_t launch_ntt_fwd_rows(const NttArgs &a, int num_limbs, int num_z,
                                int epilogue, hipStream_t s) {
   if (num_limbs <= 0 || num_z <= 0) return hipSuccess;
   dim3 gr(kRows / kTileRows, num_limbs, num_z);
-  if (epilogue == kEpiModDown && a.blocked)
+  if (epilogue == kEpiModDownPerm)
+    hipLaunchKernelGGL((ntt_fwd_rows<kEpiModDownPerm, true>), gr, dim3(256), 0, s, a);
+  else if (epilogue == kEpiModDown && a.blocked)
     hipLaunchKernelGGL((ntt_fwd_rows<kEpiModDown, true>), gr, dim3(256), 0, s, a);
   else if (epilogue == kEpiModDown)
     hipLaunchKernelGGL((ntt_fwd_rows<kEpiModDown, false>), gr, dim3(256), 0, s, a);
@@ -2458,9 +2482,10 @@ extern "C" int chd_k_ntt_fwd_rows_moddown(
     const chd_tables *t, const chd_limb_map *m, uint32_t *const *dst,
     int num_polys, int num_limbs, const uint32_t *src, long long src_pstride,
     const uint32_t *src2, long long src2_pstride, int src2_lo, int src2_hi,
-    const uint32_t *inv_prod, const uint32_t *pad, void *stream) {
+    const uint32_t *inv_prod, const uint32_t *pad, uint32_t galois,
+    void *stream) {
   const char *who = "chd_k_ntt_fwd_rows_moddown";
-  if (!src)
+  if (!src || (galois & 1u) == 0 || galois >= 2u * kN)
     return set_error(CHD_ERR_ARG, std::string(who) + ": invalid argument");
   NttArgs a;
   if (int st = moddown_multi_args(who, t, m, dst, num_polys, num_limbs, src2,
@@ -2473,7 +2498,15 @@ extern "C" int chd_k_ntt_fwd_rows_moddown(
   a.src = src;
   a.src_pstride = src_pstride;
   a.blocked = 1;
-  hipError_t e = launch_ntt_fwd_rows(a, num_limbs, num_polys, kEpiModDown,
+  // the inverse of an odd factor modulo a power of two: each step doubles
+  // the correct low bits (3 of them for g itself)
+  uint32_t inv = galois;
+  for (int i = 0; i < 4; i++) inv *= 2u - galois * inv;
+  a.galois = galois;
+  a.galois_inv = inv & (2u * kN - 1);
+  hipError_t e = launch_ntt_fwd_rows(a, num_limbs, num_polys,
+                                     galois == 1 ? kEpiModDown
+                                                 : kEpiModDownPerm,
                                      static_cast<hipStream_t>(stream));
   if (e != hipSuccess)
     return set_error(CHD_ERR_HIP,

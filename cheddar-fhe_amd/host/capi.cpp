@@ -463,16 +463,9 @@ extern "C" int chd_hrot(const chd_context *ctx, int level, uint32_t *res_bx,
              int r = rot % num_slots;
              if (r < 0) r += num_slots;
              if (r == 0) throw cheddar::Error("HRot by 0 is not a rotation");
-             const auto &p = ctx->c->param_;
-             const size_t words =
-                 static_cast<size_t>(p.LevelToNP(level).GetNumQ()) * p.degree_;
-             cheddar::Workspace::Use use_ws(ctx->c->GetWorkspace());
-             cheddar::Scratch t(ctx->c->GetWorkspace(), 2 * words);
-             ctx->c->MultKeyV(level, {t.data(), t.data() + words, nullptr},
-                              {a_bx, a_ax, nullptr},
-                              MakeEvk(ctx, evk_bx, evk_ax, evk_beta));
-             ctx->c->PermuteV(level, {res_bx, res_ax, nullptr},
-                              {t.data(), t.data() + words, nullptr}, r);
+             ctx->c->MultKeyPermuteV(level, {res_bx, res_ax, nullptr},
+                                     {a_bx, a_ax, nullptr},
+                                     MakeEvk(ctx, evk_bx, evk_ax, evk_beta), r);
            })
 }
 

@@ -635,9 +635,10 @@ class ModSwitchHandler<uint32_t> {
   // intt_rows: when given, the first pass of the INTT (stages 15..8) of the
   // INTT limbs is already there ([polynomial][limb] of the INTT limbs,
   // column-blocked, as the key accumulation leaves it).
+  // galois: the automorphism the results are permuted by (1: none).
   void ModDownMulti(const std::vector<word *> &dst, const word *src,
                     long long src_pstride, Kind kind,
-                    word *intt_rows = nullptr) const;
+                    word *intt_rows = nullptr, uint32_t galois = 1) const;
   // The source limbs a ModDown / ModDownAndRescale of this level transforms
   // back (its INTT limbs): [*first, *first + *count), contiguous. False when
   // they include terminal limbs (then they are not contiguous) or for
@@ -826,6 +827,9 @@ class Context<uint32_t> {
               bool rescale) const;
   void RescaleV(int level, CtRef res, CtCRef a) const;
   void MultKeyV(int level, CtRef res, CtCRef a, const EvkRef &key) const;
+  // MultKeyV followed by PermuteV (HRot)
+  void MultKeyPermuteV(int level, CtRef res, CtCRef a, const EvkRef &key,
+                       int galois_amount) const;
   void PermuteV(int level, CtRef res, CtCRef a, int galois_amount) const;
   // scratch arena of this context (sized for HMult / HRot at the top level)
   Workspace *GetWorkspace() const { return ws_.get(); }
@@ -871,7 +875,8 @@ class Context<uint32_t> {
                      word *intt_a = nullptr, int intt_lo = 0) const;
   void KeySwitchDown(int level, CtRef res, const word *d, const word *cb,
                      const word *ca, const CtCRef *ta, const CtCRef *tb,
-                     const EvkRef &key, bool rescale) const;
+                     const EvkRef &key, bool rescale,
+                     uint32_t galois = 1) const;
   DeviceVector<word> p_prod_;
   std::unique_ptr<Workspace> ws_;
   // EncodeConstant(1.0) at each level's default scale, for LevelDown

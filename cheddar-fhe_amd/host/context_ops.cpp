@@ -585,9 +585,14 @@ void Context<uint32_t>::MultImaginaryUnit(Ct &res, const Ct &a) const {
 
 // Context.cpp:794-799
 void Context<uint32_t>::HConj(Ct &res, const Ct &a, const Evk &conj_key) const {
-  Ct tmp;
-  MultKey(tmp, a, conj_key);
-  PermuteConjugate(res, tmp);
+  Ct out(a.GetNP());
+  MultKeyPermuteV(param_.NPToLevel(a.GetNP()),
+                  {out.bx_.data(), out.ax_.data(), nullptr},
+                  {a.bx_.data(), a.ax_.data(), nullptr}, RefOfKey(conj_key),
+                  -1);
+  out.SetScale(a.GetScale());
+  out.SetNumSlots(a.GetNumSlots());
+  res = std::move(out);
 }
 
 // Context.cpp:801-861: Permute(MultKey(a)) + b in one PermuteAccum

@@ -205,14 +205,17 @@ typedef struct chd_switch_job {
 int chd_k_switch_cols(const chd_tables *t, const chd_limb_map *m,
                       const chd_switch_job *jobs, int num_jobs, void *stream);
 /* The second pass (stages 8..15) of chd_k_ntt_fwd_moddown_multi on
- * column-blocked input src + p * src_pstride; no dst[p] may overlap it. */
+ * column-blocked input src + p * src_pstride; no dst[p] may overlap it. The
+ * result is permuted by the automorphism galois on its way out (chd_k_permute;
+ * 1: none). */
 int chd_k_ntt_fwd_rows_moddown(const chd_tables *t, const chd_limb_map *m,
                                uint32_t *const *dst, int num_polys,
                                int num_limbs, const uint32_t *src,
                                long long src_pstride, const uint32_t *src2,
                                long long src2_pstride, int src2_lo,
                                int src2_hi, const uint32_t *inv_prod,
-                               const uint32_t *pad, void *stream);
+                               const uint32_t *pad, uint32_t galois,
+                               void *stream);
 /* The second pass of chd_k_ntt_fwd_groups (num_groups <= CHD_MAX_JOBS) from
  * column-blocked src + g * group_stride into dst[g], own limbs skipped. */
 int chd_k_ntt_fwd_rows_groups(const chd_tables *t, const chd_limb_map *m,

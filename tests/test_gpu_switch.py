@@ -62,3 +62,23 @@ def test_base_switch_shapes(chd, L, alpha, mixed):
     assert np.array_equal(host(out), _orc.mod_down(x, primes, L - 1, 16))
     ctx.rescale_poly(1, out, dev(xq))
     assert np.array_equal(host(out), _orc.mod_down(xq, main, L - 1, 16))
+
+
+@pytest.mark.parametrize("rot", [1, 2, 255, 256, 1 << 14, N // 2 - 1])
+def test_rotation_in_the_last_row_pass(chd, rot):
+    """HRot, whose automorphism runs inside ModDown's last pass, for factors
+    that move columns only, rows only and both, on primes on both sides of
+    2^30"""
+    main, aux = _primes(4, 3, True)
+    ctx = chd.Context(chd.Param(main, aux, [(i, 0) for i in range(1, 5)]))
+    r = np.random.default_rng(0x607 + rot)
+    L = 3
+    b, a = uniform_limbs(r, main[:L]), uniform_limbs(r, main[:L])
+    kb, ka = (np.stack([uniform_limbs(r, main + aux) for _ in range(2)])
+              for _ in range(2))
+    res = (zeros(L, N), zeros(L, N))
+    ctx.hrot(L - 1, res, (dev(b), dev(a)), [dev(k) for k in kb],
+             [dev(k) for k in ka], rot)
+    wb, wa = _orc.hrot(b, a, kb, ka, L, 4, main, aux, 16, rot)
+    assert np.array_equal(host(res[0]), wb)
+    assert np.array_equal(host(res[1]), wa)
