@@ -42,6 +42,7 @@ SOURCES = [
     ("csrc/bconv.hip", True, MFMA_VGPR),
     ("csrc/switch_cols.hip", True, MFMA_VGPR),
     ("csrc/elementwise.hip", True, []),
+    ("csrc/encode.hip", True, []),
     ("csrc/hmult_noalloc.hip", True, []),
     ("host/device_tables.cpp", False, []),
     ("host/memory_pool.cpp", False, []),

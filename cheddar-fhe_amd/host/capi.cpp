@@ -892,17 +892,8 @@ extern "C" int chd_encode(const chd_context *ctx, int level, int num_aux,
       !msg_im || msg_len < 1 || msg_len > ctx->c->param_.degree_ / 2 || !dst)
     return set_error(CHD_ERR_ARG, "chd_encode: invalid argument");
   CHD_TRY cheddar::StreamScope scope(static_cast<hipStream_t>(stream));
-  cheddar::Plaintext<word> pt;
-  ctx->c->encoder_.Encode(pt, level, scale, Message(msg_re, msg_im, msg_len),
-                          num_aux);
-  cheddar::HipCheck(hipMemcpyAsync(dst, pt.mx_.data(),
-                                   pt.mx_.size() * sizeof(word),
-                                   hipMemcpyDeviceToDevice,
-                                   cheddar::CurrentStream()),
-                    "hipMemcpyAsync");
-  cheddar::HipCheck(hipStreamSynchronize(cheddar::CurrentStream()),
-                    "hipStreamSynchronize");
-  return pt.GetNumSlots();
+  return ctx->c->encoder_.EncodeTo(dst, level, scale, msg_re, msg_im, 1,
+                                   msg_len, num_aux);
   CHD_CATCH("chd_encode")
 }
 
@@ -932,21 +923,9 @@ extern "C" int chd_decode(const chd_context *ctx, int level, double scale,
                num_slots <= ctx->c->param_.degree_ / 2 &&
                PaddedSlots(num_slots) == num_slots,
            {
-             const auto &p = ctx->c->param_;
-             cheddar::Plaintext<word> pt(p.LevelToNP(level), p.degree_);
-             cheddar::HipCheck(hipMemcpyAsync(pt.mx_.data(), src,
-                                              pt.mx_.size() * sizeof(word),
-                                              hipMemcpyDeviceToDevice,
-                                              cheddar::CurrentStream()),
-                               "hipMemcpyAsync");
-             pt.SetNumSlots(num_slots);
-             pt.SetScale(scale);
-             std::vector<cheddar::Complex> m;
-             ctx->c->encoder_.Decode(m, pt);
-             for (int i = 0; i < num_slots; i++) {
-               out_re[i] = m[i].real();
-               out_im[i] = m[i].imag();
-             }
+             ctx->c->encoder_.DecodeFrom(out_re, out_im, 1, num_slots,
+                                         ctx->c->param_.LevelToNP(level),
+                                         scale, src);
            })
 }
 

@@ -6,8 +6,6 @@
 #include <numeric>
 #include <climits>
 #include <cmath>
-#include <exception>
-#include <thread>
 
 #include "cheddar_amd.h"
 #include "chd_device.h"
@@ -1789,39 +1787,10 @@ HoistHandler<uint32_t>::PtMap HoistHandler<uint32_t>::EncodeMap(
     for (const auto &[g, bs_map] : hoist_map)
       for (const auto &[b, msg] : bs_map) jobs.push_back(Job{g, b, &msg, {}});
   }
-  // the host halves (special IFFT and residues) of up to `width` plaintexts
-  // run on as many threads, then their uploads and NTTs in order
-  const size_t width = std::max<size_t>(
-      1, std::min<size_t>(16, std::thread::hardware_concurrency()));
   PtMap out;
-  std::vector<std::vector<word>> mx(width);
-  std::vector<int> slots(width);
-  std::vector<std::exception_ptr> err(width);
-  for (size_t start = 0; start < jobs.size(); start += width) {
-    const size_t count = std::min(width, jobs.size() - start);
-    auto host_half = [&](size_t k) {
-      try {
-        const Job &j = jobs[start + k];
-        std::vector<Complex> padded =
-            Encoder<word>::PadToPowerOfTwo(j.msg ? *j.msg : j.rotated);
-        slots[k] = static_cast<int>(padded.size());
-        mx[k] = enc.CoefficientResidues(pt_level, pt_scale, std::move(padded),
-                                        alpha);
-      } catch (...) {
-        err[k] = std::current_exception();
-      }
-    };
-    std::vector<std::thread> threads;
-    for (size_t k = 1; k < count; k++) threads.emplace_back(host_half, k);
-    host_half(0);
-    for (std::thread &t : threads) t.join();
-    for (size_t k = 0; k < count; k++)
-      if (err[k]) std::rethrow_exception(err[k]);
-    for (size_t k = 0; k < count; k++) {
-      const Job &j = jobs[start + k];
-      Pt &pt = out[j.g].try_emplace(j.b, NPInfo(0, 0, 0)).first->second;
-      enc.EncodeResidues(pt, pt_level, pt_scale, slots[k], mx[k], alpha);
-    }
+  for (const Job &j : jobs) {
+    Pt &pt = out[j.g].try_emplace(j.b, NPInfo(0, 0, 0)).first->second;
+    enc.Encode(pt, pt_level, pt_scale, j.msg ? *j.msg : j.rotated, alpha);
   }
   return out;
 }

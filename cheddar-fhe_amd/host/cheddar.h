@@ -510,6 +510,10 @@ class NTTHandler<uint32_t> {
                       const NPInfo &np_non_intt, const DvConstView<word> &src,
                       const DvConstView<word> &src_const) const;
   const chd_tables &Tables() const { return chain_.tables(); }
+  // 2^64 mod q per prime of the tables
+  const word *MontConverter() const { return chain_.mont_converter(); }
+  // the limbs of np, in order and without gaps in memory
+  chd_limb_map LimbMapOf(const NPInfo &np) const { return Map(np); }
 
  private:
   chd_limb_map Map(const NPInfo &np) const;
@@ -727,12 +731,58 @@ class Encoder<uint32_t> {
                       int num_aux = 0) const;
   void SpecialIFFT(std::vector<Complex> &data) const;
   void SpecialFFT(std::vector<Complex> &data) const;
+  // Encode and Decode on raw memory: message value i is (re[i stride],
+  // im[i stride]) on the host, the plaintext device limbs. EncodeTo returns
+  // the padded slot count. Both synchronise the stream.
+  int EncodeTo(word *dst, int level, double scale, const double *re,
+               const double *im, int stride, int len, int num_aux) const;
+  void DecodeFrom(double *re, double *im, int stride, int slots,
+                  const NPInfo &np, double scale, const word *src) const;
 
  private:
+  // Pinned staging for one message (N / 2 complex values), which the kernels
+  // read and write in place. Lent to one call, which synchronises its
+  // stream before giving it back; at most kKept stay with the encoder.
+  class Stage {
+   public:
+    explicit Stage(const Encoder &enc);
+    ~Stage();
+    Stage(const Stage &) = delete;
+    Stage &operator=(const Stage &) = delete;
+    double *data() const { return p_; }
+    void Synchronize();
+
+   private:
+    const Encoder &enc_;
+    double *p_ = nullptr;
+    bool idle_ = false;
+  };
+  static constexpr size_t kKept = 4;
+  struct StagePool {
+    std::mutex mu;
+    std::vector<double *> free;
+    ~StagePool();
+  };
+  mutable StagePool stages_;
+  // CRT constants of one prime set: (N prod_{k != i} q_k)^-1 mod q_i, then
+  // chd_k_decode's table
+  struct CrtTable {
+    DevBuf icrt, table;
+    int width = 0;  // 0: more words than the device decoder takes
+  };
+  const CrtTable &CrtOf(const NPInfo &np) const;
+  void DecodeHost(std::vector<Complex> &message, const NPInfo &np, int slots,
+                  double scale, const word *residues) const;
   const Parameter<word> &param_;
   const NTTHandler<word> *ntt_handler_;
   const int m_;  // 2N
   std::vector<Complex> twiddle_;
+  // per stage: twiddle j of the stage of stride s at s + j, inverse then
+  // forward (device, 32768 complex values each)
+  DevBuf stage_twiddle_;
+  // built on first use of a level, kept with the encoder
+  mutable std::mutex crt_mu_;
+  mutable std::map<std::pair<int, int>, CrtTable> crt_;
 };
 
 template <typename word>

@@ -431,6 +431,37 @@ typedef struct chd_bs_args {
 int chd_k_bs_fused(const chd_tables *t, const chd_limb_map *m,
                    const chd_bs_args *args, void *stream);
 
+/* Encoder (Encode.cpp:23-246), in the host encoder's operation order.
+ * twiddles: [32768][2] doubles, entry s + j the twiddle j of the stage of
+ * stride s (inverse or forward). msg_len <= 2^log_slots <= N / 2 values
+ * msg_re / msg_im [i msg_stride] (device or pinned host memory, each value
+ * read once); all values must be finite and stay so.
+ * coef and work hold 2^log_slots complex values: coef[i] = value i of the
+ * special IFFT of the zero-padded message, divided by the slots, times
+ * scale. */
+int chd_k_encode_coefficients(double *coef, double *work, const double *msg_re,
+                              const double *msg_im, int msg_stride,
+                              int msg_len, int log_slots, double scale,
+                              const double *twiddles, void *stream);
+/* dst[l] = the truncated coefficients modulo limb l's prime (real parts from
+ * index 0, imaginary ones from N / 2, N / 2 / slots apart);
+ * mont_converter: 2^64 mod q per prime of the tables */
+int chd_k_encode_residues(const chd_tables *t, const chd_limb_map *m,
+                          const uint32_t *mont_converter, uint32_t *dst,
+                          int num_limbs, const double *coef, int log_slots,
+                          void *stream);
+/* The message out of residues r_j [limbs][N] already multiplied by
+ * (Q / q_j)^-1: centred CRT, conversion to double, division by the scale and
+ * special FFT into out_re / out_im [i out_stride]. table: limbs + 2 rows of
+ * width words (Q / q_j, Q, floor(Q / 2), little-endian), width =
+ * chd_k_decode_width(words of Q + 1) (0: too wide). work: 2^log_slots complex
+ * values; out (device or pinned host memory) may not overlap it. */
+int chd_k_decode_width(int words);
+int chd_k_decode(double *out_re, double *out_im, int out_stride, double *work,
+                 const uint32_t *residues, int limbs, const uint32_t *table,
+                 int width, int log_slots, double scale,
+                 const double *twiddles, void *stream);
+
 /* Element-wise ops over num_poly polynomials of m->num_q q limbs plus aux
  * limbs (ElementWise.cu:33-220, 600-660, Basic.cuh:169-260), canonical in
  * and out. b: per polynomial (ADD, SUB, MULT) or b[0] for every polynomial
