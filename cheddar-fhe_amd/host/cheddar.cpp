@@ -46,9 +46,10 @@ StreamScope::StreamScope(hipStream_t s) : prev_(g_stream) { g_stream = s; }
 StreamScope::~StreamScope() { g_stream = prev_; }
 
 Workspace::Workspace(size_t words) {
-  buf_.Resize(words * sizeof(uint32_t));
-  base_ = buf_.as<uint32_t>();
-  cap_ = words;
+  chunks_.resize(1);
+  chunks_[0].buf.Resize(words * sizeof(uint32_t));
+  chunks_[0].base = chunks_[0].buf.as<uint32_t>();
+  chunks_[0].cap = words;
   HipCheck(hipEventCreateWithFlags(&done_, hipEventDisableTiming),
            "hipEventCreateWithFlags");
 }
@@ -93,32 +94,70 @@ Workspace::Use::~Use() {
 }
 
 Workspace::External::External(Workspace *ws, uint32_t *base, size_t words)
-    : ws_(ws), saved_base_(ws->base_), saved_cap_(ws->cap_) {
-  AssertTrue(ws->depth_ > 0 && ws->top_ == 0 && !ws->strict_,
+    : ws_(ws),
+      saved_base_(ws->chunks_[0].base),
+      saved_cap_(ws->chunks_[0].cap) {
+  AssertTrue(ws->depth_ > 0 && ws->cur_chunk_ == 0 &&
+                 ws->chunks_[0].top == 0 && !ws->strict_,
              "Workspace: external memory needs an idle guarded workspace");
   AssertTrue(base != nullptr && (reinterpret_cast<uintptr_t>(base) & 255) == 0,
              "Workspace: external memory must be 256-byte aligned");
-  ws->base_ = base;
-  ws->cap_ = words & ~static_cast<size_t>(63);
+  ws->chunks_[0].base = base;
+  ws->chunks_[0].cap = words & ~static_cast<size_t>(63);
   ws->strict_ = true;
 }
 
 Workspace::External::~External() {
-  ws_->base_ = saved_base_;
-  ws_->cap_ = saved_cap_;
-  ws_->top_ = 0;
+  ws_->chunks_[0].base = saved_base_;
+  ws_->chunks_[0].cap = saved_cap_;
+  ws_->chunks_[0].top = 0;
   ws_->strict_ = false;
 }
 
 uint32_t *Workspace::Push(size_t words) {
   const size_t w = (words + 63) & ~static_cast<size_t>(63);  // 256-byte steps
-  if (w > cap_ - top_) return nullptr;
-  uint32_t *p = base_ + top_;
-  top_ += w;
-  return p;
+  for (size_t i = cur_chunk_;; i++) {
+    if (i > 0 && strict_) return nullptr;
+    if (i == chunks_.size() && !AddChunk(w)) return nullptr;
+    Chunk &c = chunks_[i];
+    if (w > c.cap - c.top) continue;
+    cur_chunk_ = i;
+    uint32_t *p = c.base + c.top;
+    c.top += w;
+    return p;
+  }
 }
 
-void Workspace::Pop(uint32_t *p) { top_ = static_cast<size_t>(p - base_); }
+// false where nothing may be allocated: the bound is reached, the memory is
+// not there, or the stream is being captured (a plain allocation would end
+// the capture)
+bool Workspace::AddChunk(size_t words) {
+  const size_t bytes = words * sizeof(uint32_t);
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (bytes > kMaxExtraBytes - extra_bytes_ ||
+      hipStreamIsCapturing(CurrentStream(), &st) != hipSuccess ||
+      st != hipStreamCaptureStatusNone)
+    return false;
+  Chunk c;
+  try {
+    c.buf.Resize(bytes);
+  } catch (const std::exception &) {
+    (void)hipGetLastError();  // not the next launch's failure
+    return false;
+  }
+  c.base = c.buf.as<uint32_t>();
+  c.cap = words;
+  extra_bytes_ += bytes;
+  chunks_.push_back(std::move(c));
+  return true;
+}
+
+// LIFO: p is the last temporary taken, in the last chunk in use
+void Workspace::Pop(uint32_t *p) {
+  Chunk &c = chunks_[cur_chunk_];
+  c.top = static_cast<size_t>(p - c.base);
+  while (cur_chunk_ > 0 && chunks_[cur_chunk_].top == 0) cur_chunk_--;
+}
 
 Scratch::Scratch(Workspace *ws, size_t words) {
   if (words == 0) return;

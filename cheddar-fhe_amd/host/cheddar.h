@@ -303,6 +303,11 @@ void CopyDeviceToDevice(DeviceVector<word> &dst,
 // one stream at a time: a call on a different stream than the previous call
 // first makes its stream wait for the event recorded at the end of that call.
 // Calls from several host threads are serialised by a mutex.
+// A call that needs more than the arena adds a chunk, which stays (at most
+// kMaxExtraBytes of them): stream-ordered memory goes back to the system at
+// the next synchronisation and is mapped again by the next call (a hoisted
+// 28 x 28 step transform, 0.8 GiB, 1.2 ms of 4.2 per call between
+// synchronisations).
 class Workspace {
  public:
   explicit Workspace(size_t words);
@@ -336,20 +341,28 @@ class Workspace {
     uint32_t *saved_base_;
     size_t saved_cap_;
   };
-  // nullptr when the arena has no room left
+  // nullptr when there is no room and none may be added
   uint32_t *Push(size_t words);
   void Pop(uint32_t *p);
-  size_t Capacity() const { return cap_; }
+  size_t Capacity() const { return chunks_[0].cap; }
   // no fallback allocation allowed (an External guard is active)
   bool Strict() const { return strict_; }
 
  private:
+  static constexpr size_t kMaxExtraBytes = size_t{2} << 30;
+  struct Chunk {
+    DevBuf buf;  // empty while External lends memory
+    uint32_t *base = nullptr;
+    size_t cap = 0, top = 0;  // words
+  };
   void Enter();
   void Leave() noexcept;
-  DevBuf buf_;
-  uint32_t *base_ = nullptr;
+  bool AddChunk(size_t words);
+  // the arena, then the added chunks; temporaries are taken from chunk
+  // cur_chunk_ and later ones only, so releases stay in LIFO order
+  std::vector<Chunk> chunks_;
+  size_t cur_chunk_ = 0, extra_bytes_ = 0;
   bool strict_ = false;
-  size_t cap_ = 0, top_ = 0;
   int depth_ = 0;
   hipEvent_t done_ = nullptr;
   hipStream_t cur_ = nullptr, last_ = nullptr;
