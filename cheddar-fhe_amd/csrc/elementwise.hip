@@ -256,17 +256,19 @@ __global__ __launch_bounds__(kThreads) void bs_fused_kernel(chd_tables t,
   const size_t loff = static_cast<size_t>(li.l) << kLogN;
   const int c0 = blockIdx.x * kCoefPerBlock + threadIdx.x * kPerThread;
   uint32_t u[CHD_MAX_BS_GROUPS][4];
+  uint32_t own[4] = {0, 0, 0, 0};  // the input's limb (q limbs)
   for (int g = 0; g < a.beta; g++) {
     const int own_lo = group_lo(g, a.alpha, a.group_shift);
     const int own_hi = group_hi(g, a.alpha, a.group_shift, a.num_q);
-    const uint32_t *src = (li.l >= own_lo && li.l < own_hi)
-                              ? a.d + loff
-                              : a.modup + g * a.group_stride + loff;
+    const bool is_own = li.l >= own_lo && li.l < own_hi;
+    const uint32_t *src =
+        is_own ? a.d + loff : a.modup + g * a.group_stride + loff;
     const uint4 v = ld4(src + c0);
-    u[g][0] = v.x;
-    u[g][1] = v.y;
-    u[g][2] = v.z;
-    u[g][3] = v.w;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      u[g][i] = get(v, i);
+      own[i] = is_own ? u[g][i] : own[i];
+    }
   }
   uint32_t pb[4] = {0, 0, 0, 0};
   if (!li.aux) {
@@ -277,6 +279,19 @@ __global__ __launch_bounds__(kThreads) void bs_fused_kernel(chd_tables t,
     pb[1] = mont_mul(static_cast<int32_t>(v.y), pp, li.q, li.qinv);
     pb[2] = mont_mul(static_cast<int32_t>(v.z), pp, li.q, li.qinv);
     pb[3] = mont_mul(static_cast<int32_t>(v.w), pp, li.q, li.qinv);
+  }
+  if (a.dst0_b != nullptr) {
+    // baby step 0 from the words already here (two constant products and two
+    // fills of its own took 19 us at 13 + 8 limbs)
+    uint32_t pa[4] = {0, 0, 0, 0};
+    if (!li.aux) {
+      const int32_t pp = static_cast<int32_t>(a.p_prod[li.l]);
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        pa[i] = mont_mul(static_cast<int32_t>(own[i]), pp, li.q, li.qinv);
+    }
+    st4(a.dst0_b + loff + c0, make_uint4(pb[0], pb[1], pb[2], pb[3]));
+    st4(a.dst0_a + loff + c0, make_uint4(pa[0], pa[1], pa[2], pa[3]));
   }
   const size_t koff = loff + (li.aux ? a.key_gap : 0);
   const uint32_t qn = 0u - static_cast<uint32_t>(li.qinv);
@@ -744,7 +759,8 @@ extern "C" int chd_k_bs_fused(const chd_tables *t, const chd_limb_map *m,
                     args->num_q) ||
       !args->modup || !args->d ||
       !args->ct_b || !args->p_prod || args->num_q != m->num_q ||
-      m->skip_len != 0)
+      m->skip_len != 0 ||
+      (args->dst0_b == nullptr) != (args->dst0_a == nullptr))
     return set_error(CHD_ERR_ARG, "chd_k_bs_fused: invalid argument");
   for (int k = 0; k < args->num_rot; k++) {
     if (!args->dst_b[k] || !args->dst_a[k] || (args->galois[k] & 1u) == 0 ||

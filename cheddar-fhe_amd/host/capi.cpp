@@ -562,8 +562,7 @@ struct chd_hoist {
   std::unique_ptr<cheddar::LinearTransform<word>> lt;
   const cheddar::HoistHandler<word> *h = nullptr;  // own's or lt's
   int level;
-  // buffers kept across runs: the input copy, the baby steps, the result
-  cheddar::Ciphertext<word> in, res;
+  // the baby steps, kept across runs
   std::map<int, cheddar::Ciphertext<word>> babies;
 };
 
@@ -650,32 +649,19 @@ int HoistRun(const char *name, const chd_hoist *h, uint32_t *res_bx,
       key_beta < 1 || (num_keys > 0 && (!key_rot || !key_bx || !key_ax)))
     return set_error(CHD_ERR_ARG, std::string(name) + ": invalid argument");
   CHD_TRY cheddar::StreamScope scope(static_cast<hipStream_t>(stream));
-  const auto &p = h->c->param_;
   chd_context view{h->c};
   const auto keys = Keys(&view, num_keys, key_rot, key_bx, key_ax, key_beta);
   chd_hoist *m = const_cast<chd_hoist *>(h);  // buffers, not the handler
-  if (!(m->in.GetNP() == p.LevelToNP(h->level)) || m->in.bx_.size() == 0)
-    m->in = cheddar::Ciphertext<word>(p.LevelToNP(h->level));
-  const size_t in_bytes = m->in.bx_.size() * sizeof(word);
-  cheddar::HipCheck(hipMemcpyAsync(m->in.bx_.data(), ct_bx, in_bytes,
-                                   hipMemcpyDeviceToDevice,
-                                   cheddar::CurrentStream()),
-                    "hipMemcpyAsync");
-  cheddar::HipCheck(hipMemcpyAsync(m->in.ax_.data(), ct_ax, in_bytes,
-                                   hipMemcpyDeviceToDevice,
-                                   cheddar::CurrentStream()),
-                    "hipMemcpyAsync");
-  h->h->BabyStep(*h->c, m->babies, m->in, keys, min_ks);
-  h->h->GiantStep(*h->c, m->res, m->babies, keys, min_ks);
-  const size_t bytes = m->res.bx_.size() * sizeof(word);
-  cheddar::HipCheck(hipMemcpyAsync(res_bx, m->res.bx_.data(), bytes,
-                                   hipMemcpyDeviceToDevice,
-                                   cheddar::CurrentStream()),
-                    "hipMemcpyAsync");
-  cheddar::HipCheck(hipMemcpyAsync(res_ax, m->res.ax_.data(), bytes,
-                                   hipMemcpyDeviceToDevice,
-                                   cheddar::CurrentStream()),
-                    "hipMemcpyAsync");
+  // a fresh ciphertext's scale and slots: the raw result carries neither
+  const cheddar::Ciphertext<word> plain;
+  h->h->BabyStep(*h->c, m->babies,
+                 cheddar::HoistHandler<word>::Input{{ct_bx, ct_ax, nullptr},
+                                                    plain.GetScale(),
+                                                    plain.GetNumSlots()},
+                 keys, min_ks);
+  h->h->GiantStep(*h->c,
+                  cheddar::Context<word>::CtRef{res_bx, res_ax, nullptr},
+                  m->babies, keys, min_ks);
   return chd::check_launch(name);
   }
   catch (const std::exception &e) {

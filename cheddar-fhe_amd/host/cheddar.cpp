@@ -2040,26 +2040,26 @@ void HRotV(const Context<uint32_t> &ctx, int level, uint32_t *res_b,
 // Hoist.cu:517-537: bs[0] = input, bs[k s] = HRot(bs[(k - 1) s], s)
 void HoistHandler<uint32_t>::MinKSBabyStep(const Context<word> &ctx,
                                            std::map<int, Ct> &bs,
-                                           const Ct &input,
+                                           const Input &input,
                                            const KeyLookup &key_of) const {
   const int bs_stride = CheckStrideMinKS().first;
-  const NPInfo np = input.GetNP();
+  const NPInfo np = ctx.param_.LevelToNP(pt_level_);
   const size_t bytes = static_cast<size_t>(np.GetNumQ()) *
                        ctx.param_.degree_ * sizeof(word);
   auto slot = [&](int idx) -> Ct & {
     Ct &ct = bs.try_emplace(idx, np).first->second;
     if (!(ct.GetNP() == np) || ct.HasRx()) ct = Ct(np);
-    ct.SetScale(input.GetScale());
-    ct.SetNumSlots(input.GetNumSlots());
+    ct.SetScale(input.scale);
+    ct.SetNumSlots(input.slots);
     return ct;
   };
   for (int b : bs_indices_) {
     Ct &out = slot(b);
     if (b == 0) {
-      HipCheck(hipMemcpyAsync(out.bx_.data(), input.bx_.data(), bytes,
+      HipCheck(hipMemcpyAsync(out.bx_.data(), input.ct.bx, bytes,
                               hipMemcpyDeviceToDevice, CurrentStream()),
                "hipMemcpyAsync");
-      HipCheck(hipMemcpyAsync(out.ax_.data(), input.ax_.data(), bytes,
+      HipCheck(hipMemcpyAsync(out.ax_.data(), input.ct.ax, bytes,
                               hipMemcpyDeviceToDevice, CurrentStream()),
                "hipMemcpyAsync");
       continue;
@@ -2076,9 +2076,10 @@ void HoistHandler<uint32_t>::MinKSBabyStep(const Context<word> &ctx,
 // Hoist.cu:539-566: giant steps from the last down, each accumulation added
 // to the rotated running sum (PAccum with inplace), HRot by the giant-step
 // stride unless at giant step 0, then Rescale
-void HoistHandler<uint32_t>::MinKSGiantStep(const Context<word> &ctx, Ct &res,
-                                            const std::map<int, Ct> &bs,
-                                            const KeyLookup &key_of) const {
+int HoistHandler<uint32_t>::MinKSGiantStep(const Context<word> &ctx,
+                                           Context<word>::CtRef res,
+                                           const std::map<int, Ct> &bs,
+                                           const KeyLookup &key_of) const {
   const int gs_stride = CheckStrideMinKS().second;
   const Parameter<word> &param = ctx.param_;
   const int n = param.degree_;
@@ -2153,28 +2154,32 @@ void HoistHandler<uint32_t>::MinKSGiantStep(const Context<word> &ctx, Ct &res,
     first = false;
     prev = g;
   }
-  const NPInfo out_np = param.LevelToNP(pt_level_ - 1);
-  if (!(res.GetNP() == out_np) ||
-      res.bx_.size() != static_cast<size_t>(out_np.GetNumTotal()) * n ||
-      res.HasRx())
-    res = Ct(out_np);
-  ctx.RescaleV(pt_level_, {res.bx_.data(), res.ax_.data(), nullptr},
-               {acc.data(), acc.data() + qw, nullptr});
-  res.SetNumSlots(num_slots);
-  res.SetScale(pt_scale_ * ref.GetScale() /
-               param.GetRescalePrimeProd(pt_level_));
+  ctx.RescaleV(pt_level_, res, {acc.data(), acc.data() + qw, nullptr});
+  return num_slots;
 }
 
 void HoistHandler<uint32_t>::BabyStep(const Context<word> &ctx,
                                       std::map<int, Ct> &bs, const Ct &input,
                                       const KeyLookup &key_of,
                                       bool min_ks) const {
-  const Parameter<word> &param = ctx.param_;
-  const int n = param.degree_;
-  const NPInfo in_np = input.GetNP();
-  AssertTrue(in_np == param.LevelToNP(pt_level_),
+  AssertTrue(input.GetNP() == ctx.param_.LevelToNP(pt_level_),
              "Hoist: input level mismatch");
   AssertTrue(!input.HasRx(), "Hoist: input should be relinearized");
+  BabyStep(ctx, bs,
+           Input{{input.bx_.data(), input.ax_.data(), nullptr},
+                 input.GetScale(),
+                 input.GetNumSlots()},
+           key_of, min_ks);
+}
+
+void HoistHandler<uint32_t>::BabyStep(const Context<word> &ctx,
+                                      std::map<int, Ct> &bs,
+                                      const Input &input,
+                                      const KeyLookup &key_of,
+                                      bool min_ks) const {
+  const Parameter<word> &param = ctx.param_;
+  const int n = param.degree_;
+  const NPInfo in_np = param.LevelToNP(pt_level_);
   // the reference requires an empty bs; here bs may also hold the baby
   // steps of an earlier call, whose buffers are reused when their primes
   // match (no allocation in repeated evaluations)
@@ -2208,9 +2213,10 @@ void HoistHandler<uint32_t>::BabyStep(const Context<word> &ctx,
     Scratch tmp(ws, ms.ModUpScratchWords());
     word *d[CHD_MAX_BS_GROUPS];
     for (int g = 0; g < beta; g++) d[g] = buf.data() + g * gs;
-    ms.ModUpGroups(d, input.ax_.data(), tmp.data());
+    ms.ModUpGroups(d, input.ct.ax, tmp.data());
   }
-  // 2. baby step 0: the PseudoModUp of (b, a), zero on the aux limbs
+  // 2. baby step 0: the PseudoModUp of (b, a), zero on the aux limbs; with
+  // other baby steps the first fused launch below forms it too
   auto slot = [&](int idx) -> Ct & {
     Ct &ct = bs.try_emplace(idx, ext_np).first->second;
     if (!(ct.GetNP() == ext_np) ||
@@ -2218,17 +2224,22 @@ void HoistHandler<uint32_t>::BabyStep(const Context<word> &ctx,
       ct = Ct(ext_np);
     return ct;
   };
+  Ct *b0 = nullptr;
   if (bs_indices_.count(0) != 0) {
-    Ct &b0 = slot(0);
-    b0.SetScale(input.GetScale());
-    b0.SetNumSlots(input.GetNumSlots());
-    for (DeviceVector<word> *v : {&b0.bx_, &b0.ax_}) {
-      DvView<word> q_part(v->data(), num_q * n, 0);
-      const DeviceVector<word> &src = v == &b0.bx_ ? input.bx_ : input.ax_;
-      ms.PseudoModUp(q_part, src.ConstView(), p_prod);
-      K(chd_k_zero(v->data() + static_cast<size_t>(num_q) * n,
-                   static_cast<long long>(alpha) * n, CurrentStream()));
-    }
+    b0 = &slot(0);
+    b0->SetScale(input.scale);
+    b0->SetNumSlots(input.slots);
+    if (rots.empty())
+      for (DeviceVector<word> *v : {&b0->bx_, &b0->ax_}) {
+        DvView<word> q_part(v->data(), num_q * n, 0);
+        ms.PseudoModUp(q_part,
+                       DvConstView<word>(v == &b0->bx_ ? input.ct.bx
+                                                       : input.ct.ax,
+                                         num_q * n, 0),
+                       p_prod);
+        K(chd_k_zero(v->data() + static_cast<size_t>(num_q) * n,
+                     static_cast<long long>(alpha) * n, CurrentStream()));
+      }
   }
   // 3. the other baby steps, CHD_MAX_BS per fused launch
   const int prime_offset = param.GetMaxNumTer() - in_np.num_ter_;
@@ -2245,9 +2256,13 @@ void HoistHandler<uint32_t>::BabyStep(const Context<word> &ctx,
     a.group_shift = ms.GroupShift();
     a.modup = buf.data();
     a.group_stride = gs;
-    a.d = input.ax_.data();
-    a.ct_b = input.bx_.data();
+    a.d = input.ct.ax;
+    a.ct_b = input.ct.bx;
     a.p_prod = p_prod.data();
+    if (base == 0 && b0 != nullptr) {
+      a.dst0_b = b0->bx_.data();
+      a.dst0_a = b0->ax_.data();
+    }
     const int cnt = static_cast<int>(std::min<size_t>(CHD_MAX_BS, rots.size() - base));
     a.num_rot = cnt;
     for (int k = 0; k < cnt; k++) {
@@ -2271,8 +2286,8 @@ void HoistHandler<uint32_t>::BabyStep(const Context<word> &ctx,
       // scatter with the inverse automorphism (Hoist.cu:290-300)
       a.galois[k] = static_cast<uint32_t>(param.GetGaloisFactor(n / 2 - r));
       Ct &out = slot(r);
-      out.SetScale(input.GetScale());
-      out.SetNumSlots(input.GetNumSlots());
+      out.SetScale(input.scale);
+      out.SetNumSlots(input.slots);
       a.dst_b[k] = out.bx_.data();
       a.dst_a[k] = out.ax_.data();
     }
@@ -2290,12 +2305,35 @@ void HoistHandler<uint32_t>::GiantStep(const Context<word> &ctx, Ct &res,
                                        const KeyLookup &key_of,
                                        bool min_ks) const {
   const Parameter<word> &param = ctx.param_;
+  AssertTrue(!bs.empty(), "Hoist: bs should not be empty");
+  const double scale = pt_scale_ * bs.begin()->second.GetScale() /
+                       param.GetRescalePrimeProd(pt_level_);
+  // res's own buffers when they already have the output's primes
+  const NPInfo out_np = param.LevelToNP(pt_level_ - 1);
+  Ct fresh(NPInfo(0, 0, 0));
+  const bool reuse =
+      res.GetNP() == out_np && !res.HasRx() &&
+      res.bx_.size() ==
+          static_cast<size_t>(out_np.GetNumTotal()) * param.degree_;
+  if (!reuse) fresh = Ct(out_np);
+  Ct &out = reuse ? res : fresh;
+  const int slots = GiantStep(
+      ctx, Context<word>::CtRef{out.bx_.data(), out.ax_.data(), nullptr}, bs,
+      key_of, min_ks);
+  if (!reuse) res = std::move(fresh);
+  res.SetNumSlots(slots);
+  res.SetScale(scale);
+}
+
+int HoistHandler<uint32_t>::GiantStep(const Context<word> &ctx,
+                                      Context<word>::CtRef res,
+                                      const std::map<int, Ct> &bs,
+                                      const KeyLookup &key_of,
+                                      bool min_ks) const {
+  const Parameter<word> &param = ctx.param_;
   const int n = param.degree_;
   AssertTrue(!bs.empty(), "Hoist: bs should not be empty");
-  if (min_ks) {
-    MinKSGiantStep(ctx, res, bs, key_of);
-    return;
-  }
+  if (min_ks) return MinKSGiantStep(ctx, res, bs, key_of);
   const Ct &ref = bs.begin()->second;
   const NPInfo ext_np = ref.GetNP();
   const int alpha = param.alpha_;
@@ -2306,7 +2344,6 @@ void HoistHandler<uint32_t>::GiantStep(const Context<word> &ctx, Ct &res,
   const int num_q = ext_np.GetNumQ();
   const int total = num_q + alpha;
   const size_t tw = static_cast<size_t>(total) * n;
-  const double input_scale = ref.GetScale();
   int num_slots = ref.GetNumSlots();
   for (const auto &[g, pmap] : pt_map_)
     for (const auto &[b, pt] : pmap) {
@@ -2425,18 +2462,10 @@ void HoistHandler<uint32_t>::GiantStep(const Context<word> &ctx, Ct &res,
                           CurrentStream()));
     first = false;
   }
-  // EvaluateFinalModDown: merged ModDown and rescale of both polynomials,
-  // into res's own buffers when they already have the output's primes
-  const NPInfo out_np = param.LevelToNP(pt_level_ - 1);
-  if (!(res.GetNP() == out_np) ||
-      res.bx_.size() != static_cast<size_t>(out_np.GetNumTotal()) * n ||
-      res.HasRx())
-    res = Ct(out_np);
-  ms.ModDownMulti({res.bx_.data(), res.ax_.data()}, finp,
-                  static_cast<long long>(tw),
+  // EvaluateFinalModDown: merged ModDown and rescale of both polynomials
+  ms.ModDownMulti({res.bx, res.ax}, finp, static_cast<long long>(tw),
                   ModSwitchHandler<word>::Kind::ModDownAndRescale);
-  res.SetNumSlots(num_slots);
-  res.SetScale(pt_scale_ * input_scale / param.GetRescalePrimeProd(pt_level_));
+  return num_slots;
 }
 
 // ------------------------------------------------------- StripedMatrix --

@@ -1013,16 +1013,30 @@ class HoistHandler<uint32_t> {
   void GiantStep(const Context<word> &ctx, Ct &res,
                  const std::map<int, Ct> &bs, const KeyLookup &key,
                  bool min_ks = false) const;
+  // the same on raw polynomials: the input's are read by BabyStep alone,
+  // the result's written by GiantStep's last launch (so they may be the
+  // input's); returns the result's slot count
+  struct Input {
+    Context<word>::CtCRef ct;  // num_q limbs at the plaintexts' level
+    double scale;
+    int slots;
+  };
+  void BabyStep(const Context<word> &ctx, std::map<int, Ct> &bs,
+                const Input &input, const KeyLookup &key,
+                bool min_ks = false) const;
+  int GiantStep(const Context<word> &ctx, Context<word>::CtRef res,
+                const std::map<int, Ct> &bs, const KeyLookup &key,
+                bool min_ks = false) const;
 
  private:
   int pt_level_;
   double pt_scale_;
   std::pair<int, int> CheckStrideMinKS() const;
   void MinKSBabyStep(const Context<word> &ctx, std::map<int, Ct> &bs,
-                     const Ct &input, const KeyLookup &key_of) const;
-  void MinKSGiantStep(const Context<word> &ctx, Ct &res,
-                      const std::map<int, Ct> &bs,
-                      const KeyLookup &key_of) const;
+                     const Input &input, const KeyLookup &key_of) const;
+  int MinKSGiantStep(const Context<word> &ctx, Context<word>::CtRef res,
+                     const std::map<int, Ct> &bs,
+                     const KeyLookup &key_of) const;
   static PtMap EncodeMap(const Context<word> &context,
                          const PlainHoistMap &hoist_map, int pt_level,
                          double pt_scale, bool suppress_bs_swap);

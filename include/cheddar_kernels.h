@@ -427,6 +427,9 @@ typedef struct chd_bs_args {
   uint32_t galois[CHD_MAX_BS];
   uint32_t *dst_b[CHD_MAX_BS];
   uint32_t *dst_a[CHD_MAX_BS];
+  /* when set (both), baby step 0 as well: MontMul((ct_b, d), p_prod) on the q
+   * limbs, zero on the aux limbs */
+  uint32_t *dst0_b, *dst0_a;
 } chd_bs_args;
 int chd_k_bs_fused(const chd_tables *t, const chd_limb_map *m,
                    const chd_bs_args *args, void *stream);
