@@ -21,10 +21,13 @@
 //            applied as MontMul(x, c) (NTT.cu:23-229, 673-813).
 // Arithmetic. Primes below 2^30 use unsigned lazy butterflies whose
 // Montgomery product is the 64-bit multiply-add form (three instructions,
-// mont_mad); primes in [2^30, 2^31) use the reference's signed lazy
-// butterfly (NTTUtils.cuh:19-60) in Montgomery-Shoup form, MontMul(b, w) =
-// mulhi(b, w) - mulhi(b w' mod 2^32, q) with w' = w q^-1. The per-twiddle
-// companion (w (-q^-1) or w q^-1) is derived on the fly: one multiply per
+// mont_mad). In [2^30, 2^31) 4q does not fit 32 bits: the same product, with
+// both butterfly inputs (forward) or outputs (inverse) reduced instead, nine
+// instructions where the lazy form takes seven. The reference's signed
+// butterfly (NTTUtils.cuh:19-60) takes ten or eleven: with it the single pass
+// took 19.0 us for 64 limbs of such primes (32: 18.5) and takes 16.3 (15.7),
+// the two passes 19.0 (13.3) and 18.0 (12.8).
+// The per-twiddle companion w (-q^-1) is derived on the fly: one multiply per
 // twiddle, scalar when the twiddle is wave-uniform.
 #include <algorithm>
 #include <type_traits>
@@ -69,47 +72,11 @@ __device__ __forceinline__ int32_t mont(int32_t b, int32_t w, int32_t wq,
   return hi - __mulhi(t, q);
 }
 
-// the same for a per-lane twiddle, without the companion w q^-1: b w as one
-// 64-bit product (v_mad_i64_i32), t = (b w mod 2^32) q^-1
-__device__ __forceinline__ int32_t mont_s(int32_t b, int32_t w, uint32_t qinv,
-                                          int32_t q) {
-  const int64_t p = static_cast<int64_t>(b) * w;
-  const int32_t t =
-      static_cast<int32_t>(static_cast<uint32_t>(p) * qinv);
-  return static_cast<int32_t>(p >> 32) - __mulhi(t, q);
-}
-
 // [-q, q) -> [0, q) with one add and an unsigned min
 __device__ __forceinline__ int32_t norm(int32_t a, int32_t q) {
   uint32_t ua = static_cast<uint32_t>(a);
   uint32_t uq = ua + static_cast<uint32_t>(q);
   return static_cast<int32_t>(ua < uq ? ua : uq);
-}
-
-// ButterflyNTT (NTTUtils.cuh:19-34): a, b in [-q, q); m = MontMul(b, w)
-__device__ __forceinline__ void ct_bfly_m(int32_t &a, int32_t &b, int32_t m,
-                                          int32_t q) {
-  m = norm(m, q);
-  int32_t an = norm(a, q);
-  b = an - m;
-  a = (an - q) + m;
-}
-__device__ __forceinline__ void ct_bfly(int32_t &a, int32_t &b, int32_t w,
-                                        int32_t wq, int32_t q) {
-  ct_bfly_m(a, b, mont(b, w, wq, q), q);
-}
-
-// ButterflyINTT (NTTUtils.cuh:46-60); returns an - bn for the product
-__device__ __forceinline__ int32_t gs_bfly_sum(int32_t &a, int32_t b,
-                                               int32_t q) {
-  int32_t an = norm(a, q);
-  int32_t bn = norm(b, q);
-  a = (an - q) + bn;
-  return an - bn;
-}
-__device__ __forceinline__ void gs_bfly(int32_t &a, int32_t &b, int32_t w,
-                                        int32_t wq, int32_t q) {
-  b = mont(gs_bfly_sum(a, b, q), w, wq, q);
 }
 
 // Lazy butterflies for q < 2^30 (4q < 2^32), unsigned values: CT keeps
@@ -175,6 +142,23 @@ __device__ __forceinline__ uint32_t gs_lazy_sum(uint32_t &a, uint32_t b,
 __device__ __forceinline__ void gs_lazy(uint32_t &a, uint32_t &b, uint32_t w,
                                         uint32_t wn, uint32_t q) {
   b = mont_mad(gs_lazy_sum(a, b, q), w, wn, q);  // [0, 2q)
+}
+
+// q < 2^31. CT: a in [0, 2q), d = b w 2^-32 in [0, 2q) -> a + d, a - d in
+// [0, 2q)
+__device__ __forceinline__ void ct_wide_d(uint32_t &a, uint32_t &b, uint32_t d,
+                                          uint32_t q) {
+  const uint32_t ar = umin(a, a - q), dr = umin(d, d - q);  // [0, q)
+  b = sad(q, dr, ar);
+  a = ar + dr;
+}
+// GS: a, b in [0, q) -> a + b in [0, q); returns a - b in (0, 2q)
+__device__ __forceinline__ uint32_t gs_wide_sum(uint32_t &a, uint32_t b,
+                                                uint32_t q) {
+  const uint32_t s = a + b;
+  const uint32_t t = sad(q, b, a);
+  a = umin(s, s - q);
+  return t;
 }
 
 // [0, 4q) -> [0, q)
@@ -336,16 +320,15 @@ __device__ __forceinline__ u32x4 blocked_lds4(const uint32_t *xt, int v) {
 }
 
 // Per-limb arithmetic policy. Values between the two passes of a transform
-// stay unreduced in the policy's range: [0, 4q) (forward, lazy), [0, 2q)
-// (inverse, lazy) or [-q, q) (reference form, any q < 2^31).
+// stay unreduced in the policy's range: [0, 4q) (forward) and [0, 2q)
+// (inverse) for q < 2^30, [0, 2q) and [0, q) for q < 2^31.
 template <bool kLazy>
 struct Arith;
 
-// twq(w) is the per-twiddle companion of w that ct / gs / mul take:
-// w (-q^-1) for the lazy form, w q^-1 for the reference form. Wave-uniform
-// twiddles use it (a scalar multiply); per-lane twiddles use ctv / gsv,
-// which derive the Montgomery factor from the product instead.
-// ct<false> skips the reduction of a, for a known to lie in [0, 2q).
+// twq(w) = w (-q^-1) is the per-twiddle companion of w that ct / gs / mul
+// take. Wave-uniform twiddles use it (a scalar multiply); per-lane twiddles
+// use ctv / gsv, which derive the Montgomery factor from the product instead.
+// ct<false> skips the reduction of a to [0, 2q), for a known to lie there.
 template <>
 struct Arith<true> {
   using T = uint32_t;
@@ -377,41 +360,39 @@ struct Arith<true> {
 
 template <>
 struct Arith<false> {
-  using T = int32_t;
-  int32_t q;
-  uint32_t qinv;
-  __device__ Arith(uint32_t q_, uint32_t qinv_)
-      : q(static_cast<int32_t>(q_)), qinv(qinv_) {}
-  __device__ uint32_t twq(uint32_t w) const { return w * qinv; }
+  using T = uint32_t;
+  uint32_t q;
+  uint32_t qn;  // -q^-1 mod 2^32
+  __device__ Arith(uint32_t q_, uint32_t qinv) : q(q_), qn(0u - qinv) {}
+  __device__ uint32_t twq(uint32_t w) const { return w * qn; }
   template <bool kRed = true>
-  __device__ void ct(T &a, T &b, uint32_t w, uint32_t wq) const {
-    ct_bfly(a, b, static_cast<int32_t>(w), static_cast<int32_t>(wq), q);
+  __device__ void ct(T &a, T &b, uint32_t w, uint32_t wn) const {
+    ct_wide_d(a, b, mont_mad(b, w, wn, q), q);
   }
   template <bool kRed = true>
   __device__ void ctv(T &a, T &b, uint32_t w) const {
-    ct_bfly_m(a, b, mont_s(b, static_cast<int32_t>(w), qinv, q), q);
+    ct_wide_d(a, b, mont_lo(b, w, qn, q), q);
   }
-  __device__ void gs(T &a, T &b, uint32_t w, uint32_t wq) const {
-    gs_bfly(a, b, static_cast<int32_t>(w), static_cast<int32_t>(wq), q);
+  __device__ void gs(T &a, T &b, uint32_t w, uint32_t wn) const {
+    const uint32_t d = mont_mad(gs_wide_sum(a, b, q), w, wn, q);
+    b = umin(d, d - q);
   }
   __device__ void gsv(T &a, T &b, uint32_t w) const {
-    b = mont_s(gs_bfly_sum(a, b, q), static_cast<int32_t>(w), qinv, q);
+    const uint32_t d = mont_lo(gs_wide_sum(a, b, q), w, qn, q);
+    b = umin(d, d - q);
   }
-  __device__ T mul(T x, uint32_t c, uint32_t cq) const {
-    return mont(x, static_cast<int32_t>(c), static_cast<int32_t>(cq), q);
+  // MontMul(x, c) for any x, result in [0, 2q)
+  __device__ T mul(T x, uint32_t c, uint32_t cn) const {
+    return mont_mad(x, c, cn, q);
   }
-  __device__ uint32_t canon_fwd(T x) const {
-    return static_cast<uint32_t>(norm(x, q));
-  }
-  __device__ uint32_t canon_inv(T x) const {
-    return static_cast<uint32_t>(norm(x, q));
-  }
+  __device__ uint32_t canon_fwd(T x) const { return umin(x, x - q); }
+  __device__ uint32_t canon_inv(T x) const { return umin(x, x - q); }
 };
 
 // ------------------------------------------------------------------------
 // Kernel skeleton: each kernel decodes its limb, issues the data loads of the
 // whole tile first (they depend on kernel arguments only), then reads the
-// prime and twiddles and branches to the lazy (q < 2^30) or reference-form
+// prime and twiddles and branches to the lazy (q < 2^30) or the wide (q < 2^31)
 // body. Twiddles of both half-passes are fetched before the LDS barrier.
 // ------------------------------------------------------------------------
 
@@ -1258,6 +1239,18 @@ __device__ __forceinline__ void phase_mark(int slot) {
 #define CHD_PHASE(k)
 #endif
 
+// Polynomial of item li of a single pass: li / num_limbs, from
+// rcp = floor(2^32 / num_limbs) + 1 (0 for one limb; exact while li
+// num_limbs < 2^32). The division itself is a vector sequence whose result
+// stays in vector registers with all that follows from it: every buffer
+// resource was then read back in a loop around each load (13.5 -> 20.8 us
+// for 32 limbs, once the two arithmetics below had the same shape).
+__device__ __forceinline__ int item_poly(int li, int num_limbs, uint32_t rcp) {
+  return num_limbs == 1
+             ? li
+             : static_cast<int>(__umulhi(static_cast<uint32_t>(li), rcp));
+}
+
 constexpr int kQuarter = kN / 4;
 constexpr int kQLdsWords = kQuarter + kQuarter / 16;  // 4 pad words per 64
 __device__ __forceinline__ int qidx(int n) { return n + ((n >> 6) << 2); }
@@ -1336,6 +1329,10 @@ __device__ __forceinline__ void fwd_1p_body(const NttArgs &a, const Limb &lb,
   // workgroups read it together), default caching for a broadcast source,
   // which every workgroup of the polynomial reads and the L2 keeps for them
   constexpr int kSrcAux = kBcast ? 0 : 2;
+  // The two arithmetics start with the same loads and products, which the
+  // compiler would hoist above the branch between them, all 16 elements at
+  // once: beyond 64 VGPRs, and 15-23 of them spilled (13.5 -> 20.8 us).
+  const int t = threadIdx.x;
   const A ar(q, qinv);
   const uint32_t *tw = a.tab.tw + (static_cast<size_t>(lb.ti) << kLogN);
   const uint32_t *src =
@@ -1345,7 +1342,6 @@ __device__ __forceinline__ void fwd_1p_body(const NttArgs &a, const Limb &lb,
                   j * kQuarter;
   const rsrc_t rtw = make_rsrc(tw, 4u * kN);
   const rsrc_t rsrc = make_rsrc(src, 4u * kN);
-  const int t = threadIdx.x;
   const int lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   CHD_PHASE(0);
@@ -1401,10 +1397,14 @@ __device__ __forceinline__ void fwd_1p_body(const NttArgs &a, const Limb &lb,
   // lane's 16 go in the scalar offset
   const uint32_t vt = 4u * static_cast<uint32_t>(t);
   T x[16];
-  // ---- round 1: stages 0, 1 of quarter j (bits 15, 14), then 2..5
-  if constexpr (kLazy) {
-    // one 64-bit dot product and one reduction per output: with canonical
-    // inputs and constants below q < 2^30 the sum stays below q 2^32
+  // The scheduler otherwise mixes the address arithmetic above into the
+  // round's loads, which moves code between the two bodies and spills 4-7
+  // registers of the 64 both have. In the lazy body this barrier costs 1.2 us.
+  if constexpr (!kLazy) __builtin_amdgcn_sched_barrier(0);
+  // ---- round 1: stages 0, 1 of quarter j (bits 15, 14), then 2..5.
+  // Stages 0 and 1 are one 64-bit dot product and one reduction per output
+  // (canonical inputs and constants: below 4 q^2 < 2^64).
+  {
     const uint32_t qn = ar.qn;
     const uint32_t w01 = mont_mad(w0, w1, w1 * qn, q);
     uint32_t c[4];
@@ -1436,18 +1436,17 @@ __device__ __forceinline__ void fwd_1p_body(const NttArgs &a, const Limb &lb,
         // centred inputs of a source prime below 2^31, |x| < 2^30, times
         // constants below q: the signed sum lies in (-q 2^32, q 2^32);
         // adding q 2^32 (= 0 mod q) makes it positive and below q 2^33 <
-        // 2^63, and the reduction below then lands in [0, 3q), inside the
-        // [0, 4q) the butterflies take
-        acc = static_cast<uint64_t>(
-            (static_cast<int64_t>(q) << 32) +
-            static_cast<int64_t>(static_cast<int32_t>(x0)) *
-                static_cast<int32_t>(c[0]) +
-            static_cast<int64_t>(static_cast<int32_t>(x1)) *
-                static_cast<int32_t>(c[1]) +
-            static_cast<int64_t>(static_cast<int32_t>(x2)) *
-                static_cast<int32_t>(c[2]) +
-            static_cast<int64_t>(static_cast<int32_t>(x3)) *
-                static_cast<int32_t>(c[3]));
+        // 2^64
+        acc = (static_cast<uint64_t>(q) << 32) +
+              static_cast<uint64_t>(
+                  static_cast<int64_t>(static_cast<int32_t>(x0)) *
+                      static_cast<int32_t>(c[0]) +
+                  static_cast<int64_t>(static_cast<int32_t>(x1)) *
+                      static_cast<int32_t>(c[1]) +
+                  static_cast<int64_t>(static_cast<int32_t>(x2)) *
+                      static_cast<int32_t>(c[2]) +
+                  static_cast<int64_t>(static_cast<int32_t>(x3)) *
+                      static_cast<int32_t>(c[3]));
       } else {
         acc = static_cast<uint64_t>(x0) * c[0] +
               static_cast<uint64_t>(x1) * c[1] +
@@ -1455,39 +1454,21 @@ __device__ __forceinline__ void fwd_1p_body(const NttArgs &a, const Limb &lb,
               static_cast<uint64_t>(x3) * c[3];
       }
       const uint32_t m = static_cast<uint32_t>(acc) * qn;
-      x[k] = static_cast<uint32_t>((static_cast<uint64_t>(m) * q + acc) >> 32);
-    }
-  } else {
-    // reference-form butterflies, keeping the half of each that lies in
-    // quarter j (NTTUtils.cuh:19-34)
-    const int32_t qs = static_cast<int32_t>(q);
-    const int32_t w0s = static_cast<int32_t>(w0);
-    const int32_t w0q = static_cast<int32_t>(w0 * qinv);
-    const int32_t w1s = static_cast<int32_t>(w1);
-    const int32_t w1q = static_cast<int32_t>(w1 * qinv);
-    int32_t ce = 0, ceq = 0;
-    if constexpr (kPre) {
-      ce = static_cast<int32_t>(a.cst[lb.ci]);
-      ceq = static_cast<int32_t>(static_cast<uint32_t>(ce) * qinv);
-    }
-    const bool hi0 = j >= 2, hi1 = j & 1;
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-      const uint32_t so = 4u * static_cast<uint32_t>(k << 10);
-      int32_t xm[4];
-#pragma unroll
-      for (int m = 0; m < 4; m++) {
-        xm[m] = static_cast<int32_t>(
-            bld1<kSrcAux>(rsrc, vt, so + 4u * kQuarter * m));
-        // (a broadcast source is centred: mont takes signed inputs)
-        if constexpr (kPre) xm[m] = mont(xm[m], ce, ceq, qs);
+      if constexpr (kLazy) {
+        // the sum is below q 2^32 (broadcast: q 2^33), so this is in [0, 2q)
+        // (broadcast: [0, 3q), inside the [0, 4q) the butterflies take)
+        x[k] =
+            static_cast<uint32_t>((static_cast<uint64_t>(m) * q + acc) >> 32);
+      } else {
+        // the high word, below 2q, is reduced on its own: the 64-bit sum of
+        // both could overflow. [0, q) + [0, q] is below 2q for the words
+        // that occur (reduce_sum4)
+        const uint32_t hi = static_cast<uint32_t>(acc >> 32);
+        x[k] = umin(hi, hi - q) +
+               static_cast<uint32_t>((static_cast<uint64_t>(m) * q +
+                                      static_cast<uint32_t>(acc)) >>
+                                     32);
       }
-      ct_bfly(xm[0], xm[2], w0s, w0q, qs);
-      ct_bfly(xm[1], xm[3], w0s, w0q, qs);
-      int32_t ya = hi0 ? xm[2] : xm[0];
-      int32_t yb = hi0 ? xm[3] : xm[1];
-      ct_bfly(ya, yb, w1s, w1q, qs);
-      x[k] = hi1 ? yb : ya;
     }
   }
   CHD_PHASE(1);
@@ -1601,13 +1582,14 @@ __device__ __forceinline__ void fwd_1p_body(const NttArgs &a, const Limb &lb,
 // grid: 1D, 4 * roundup(limbs * polys, 8) blocks of 1024 threads
 template <int kEpi, bool kPre>
 __device__ __forceinline__ void fwd_1p_entry(const NttArgs &a, int num_limbs,
-                                             int num_items, uint32_t *lds) {
+                                             int num_items, uint32_t rcp,
+                                             uint32_t *lds) {
   const int b = blockIdx.x;
   const int slot = b >> 3;
   const int j = slot & 3;
   const int li = (slot >> 2) * 8 + (b & 7);
   if (li >= num_items) return;
-  const int z = li / num_limbs;
+  const int z = item_poly(li, num_limbs, rcp);
   const Limb lb = decode(a.map, li - z * num_limbs);
   const uint32_t q = a.tab.q[lb.ti];
   const uint32_t qinv = static_cast<uint32_t>(a.tab.qinv[lb.ti]);
@@ -1629,16 +1611,17 @@ __device__ __forceinline__ void fwd_1p_entry(const NttArgs &a, int num_limbs,
 #endif
 template <int kEpi, bool kPre>
 __global__ __launch_bounds__(1024) CHD_FWD_1P_WAVES
-void ntt_fwd_1p(NttArgs a, int num_limbs, int num_items) {
+void ntt_fwd_1p(NttArgs a, int num_limbs, int num_items, uint32_t rcp) {
   __shared__ __align__(16) uint32_t lds[kQLdsWords];
-  fwd_1p_entry<kEpi, kPre>(a, num_limbs, num_items, lds);
+  fwd_1p_entry<kEpi, kPre>(a, num_limbs, num_items, rcp, lds);
 }
 
 __global__ __launch_bounds__(1024) void ntt_fwd_1p_bcast(NttArgs a,
                                                          int num_limbs,
-                                                         int num_items) {
+                                                         int num_items,
+                                                         uint32_t rcp) {
   __shared__ __align__(16) uint32_t lds[kQLdsWords];
-  fwd_1p_entry<kEpiModDown, true>(a, num_limbs, num_items, lds);
+  fwd_1p_entry<kEpiModDown, true>(a, num_limbs, num_items, rcp, lds);
 }
 
 // ------------------------------------------------------------------------
@@ -1788,15 +1771,16 @@ __device__ __forceinline__ void inv_1p_body(const NttArgs &a, const Limb &lb,
           static_cast<uint32_t>((static_cast<uint64_t>(m) * q + acc) >> 32);
       x[rho] = mont_lo(d, tau[rho], qn, q);  // [0, 2q)
     } else {
-      // reference form: canonical inputs (signed ones in (-q, q) as well)
+      // canonical inputs, and signed ones in (-q, q) as well
       uint64_t acc = 0;
 #pragma unroll
       for (int i = 0; i < 4; i++)
         acc += static_cast<uint64_t>(
                    static_cast<uint32_t>(norm(static_cast<int32_t>(y[i]), qs))) *
                cc[i];
-      const int32_t d = static_cast<int32_t>(reduce_sum4(acc, q, qn));
-      x[rho] = mont_s(d, static_cast<int32_t>(tau[rho]), qinv, qs);  // (-q, q)
+      const uint32_t d = reduce_sum4(acc, q, qn);
+      const uint32_t v = mont_lo(d, tau[rho], qn, q);
+      x[rho] = umin(v, v - q);  // [0, q)
     }
   }
   T *xs = reinterpret_cast<T *>(lds);
@@ -1884,14 +1868,15 @@ __device__ __forceinline__ void inv_1p_body(const NttArgs &a, const Limb &lb,
 // classes of a limb 8 block ids apart: one XCD)
 template <int kEpi>
 __global__ __launch_bounds__(1024) void ntt_inv_1p(NttArgs a, int num_limbs,
-                                                   int num_items) {
+                                                   int num_items,
+                                                   uint32_t rcp) {
   __shared__ __align__(16) uint32_t lds[kQLdsWords];
   const int b = blockIdx.x;
   const int slot = b >> 3;
   const int s = slot & 3;
   const int li = (slot >> 2) * 8 + (b & 7);
   if (li >= num_items) return;
-  const int z = li / num_limbs;
+  const int z = item_poly(li, num_limbs, rcp);
   const Limb lb = decode(a.map, li - z * num_limbs);
   const uint32_t q = a.tab.q[lb.ti];
   const uint32_t qinv = static_cast<uint32_t>(a.tab.qinv[lb.ti]);
@@ -1935,6 +1920,11 @@ hipError_t launch_modup_keyacc(const KeyAccBatch &a, int num_jobs,
   return hipGetLastError();
 }
 
+static uint32_t item_rcp(int num_limbs) {
+  return num_limbs == 1 ? 0
+                        : static_cast<uint32_t>((1ull << 32) / num_limbs) + 1;
+}
+
 hipError_t launch_ntt_fwd(const NttArgs &a, int num_limbs, int num_polys,
                           bool pre_const, int epilogue, hipStream_t s) {
   if (num_limbs <= 0 || num_polys <= 0) return hipSuccess;
@@ -1949,16 +1939,16 @@ hipError_t launch_ntt_fwd(const NttArgs &a, int num_limbs, int num_polys,
     dim3 g1(4 * ((items + 7) / 8 * 8));
     if (epilogue == kEpiModDown && a.src_bcast)
       hipLaunchKernelGGL(ntt_fwd_1p_bcast, g1, dim3(1024), 0, s, a,
-                         num_limbs, items);
+                         num_limbs, items, item_rcp(num_limbs));
     else if (epilogue == kEpiModDown)
       hipLaunchKernelGGL((ntt_fwd_1p<kEpiModDown, false>), g1, dim3(1024), 0,
-                         s, a, num_limbs, items);
+                         s, a, num_limbs, items, item_rcp(num_limbs));
     else if (pre_const)
       hipLaunchKernelGGL((ntt_fwd_1p<kEpiStore, true>), g1, dim3(1024), 0, s,
-                         a, num_limbs, items);
+                         a, num_limbs, items, item_rcp(num_limbs));
     else
       hipLaunchKernelGGL((ntt_fwd_1p<kEpiStore, false>), g1, dim3(1024), 0, s,
-                         a, num_limbs, items);
+                         a, num_limbs, items, item_rcp(num_limbs));
     return hipGetLastError();
   }
   dim3 gc(kCols / kTileCols, num_limbs, num_polys);
@@ -2005,10 +1995,10 @@ hipError_t launch_ntt_inv(const NttArgs &a, int num_limbs, int num_polys,
     dim3 g1(4 * ((items + 7) / 8 * 8));
     if (epilogue == kEpiConstCentre)
       hipLaunchKernelGGL(ntt_inv_1p<kEpiConstCentre>, g1, dim3(1024), 0, s, a,
-                         num_limbs, items);
+                         num_limbs, items, item_rcp(num_limbs));
     else
       hipLaunchKernelGGL(ntt_inv_1p<kEpiConst>, g1, dim3(1024), 0, s, a,
-                         num_limbs, items);
+                         num_limbs, items, item_rcp(num_limbs));
     return hipGetLastError();
   }
   hipError_t e = launch_ntt_inv_rows(a, num_limbs, num_polys, s);

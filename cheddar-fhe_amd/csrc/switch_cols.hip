@@ -186,7 +186,7 @@ __device__ __forceinline__ void gs16(uint32_t (&x)[16],
 }
 
 // Inverse column stages of one column: x holds rows 16 rg + k as the inverse
-// row pass left them ([0, 2q), or signed [-q, q) for q >= 2^30); the centred
+// row pass left them (below 2q; below q for q >= 2^30); the centred
 // MontMul(x, ce), split into signed byte digits, goes to xt.
 template <bool kSmall>
 __device__ __forceinline__ void inv_column(uint32_t (&x)[16],
@@ -195,9 +195,8 @@ __device__ __forceinline__ void inv_column(uint32_t (&x)[16],
                                            uint32_t q, uint32_t qn,
                                            uint32_t ce, uint32_t *xt) {
   if constexpr (!kSmall) {
-    const uint32_t add = q >= (1u << 30) ? q : 0u - q;
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = umin(x[k], x[k] + add);
+    for (int k = 0; k < 16; k++) x[k] = umin(x[k], x[k] - q);
   }
   gs16<kSmall>(x, wl, q, qn);
 #pragma unroll
@@ -233,9 +232,6 @@ __device__ __forceinline__ void fwd_column(uint32_t (&x)[16],
 #pragma unroll
   for (int k = 0; k < 16; k++) x[k] = xt[17 * rg + k];
   ct16<kSmall, false>(x, wl, q, qn);
-  const uint32_t off = kSmall || q < (1u << 30) ? 0 : q;
-#pragma unroll
-  for (int k = 0; k < 16; k++) x[k] -= off;
 }
 
 // what a lane needs of its destination limb
