@@ -42,7 +42,18 @@ namespace {
 
 constexpr int kRows = 256;
 constexpr int kCols = 256;
-constexpr int kTileCols = 32;   // columns per column-pass workgroup
+// Columns per column-pass workgroup. The passes of a few limbs leave most of
+// the chip idle and take the latency of one workgroup, which half as many
+// columns (256 threads instead of 512) shorten: forward and back in two
+// passes each, 1 limb 8.5 + 8.3 -> 7.8 + 7.9 us, 8 limbs 9.5 + 9.1 -> 8.8 +
+// 8.7, 12 limbs 9.9 + 9.2 -> 9.5 + 9.2, 16 limbs 10.4 + 9.1 -> 10.0 + 9.8
+// (31-bit primes 11.4 + 10.4 -> 10.6 + 10.6). With more limbs the halved
+// pieces of a row cost bandwidth (24 limbs 11.5 + 10.5 against 12.8 + 12.5).
+// 8 and 4 columns are slower than 16 at every size.
+constexpr int kTileCols = 32;
+constexpr int kNarrowCols = 16;
+constexpr int kNarrowFwd = 16;  // limbs of all polynomials
+constexpr int kNarrowInv = 12;
 constexpr int kTileRows = 16;   // rows per row-pass workgroup
 constexpr int kRowPad = kCols + kCols / 16;
 
@@ -397,8 +408,8 @@ struct Arith<false> {
 // ------------------------------------------------------------------------
 
 // forward, column pass: stages 0..7 (src -> dst, dst left unreduced)
-// grid (kCols / kTileCols, limbs, polys), block 512
-template <bool kPre, bool kLazy>
+// grid (kCols / kTC, limbs, polys), block 16 kTC
+template <bool kPre, bool kLazy, int kTC>
 __device__ __forceinline__ void fwd_cols_body(const NttArgs &a, const Limb &lb,
                                               uint32_t (&xin)[16], uint32_t q,
                                               uint32_t qinv, void *dst,
@@ -407,9 +418,9 @@ __device__ __forceinline__ void fwd_cols_body(const NttArgs &a, const Limb &lb,
   using T = typename A::T;
   const A ar(q, qinv);
   const uint32_t *tw = a.tab.tw + (static_cast<size_t>(lb.ti) << kLogN);
-  const int c = threadIdx.x & (kTileCols - 1);
-  const int rg = threadIdx.x / kTileCols;  // 0..15
-  const uint32_t col = blockIdx.x * kTileCols + c;
+  const int c = threadIdx.x & (kTC - 1);
+  const int rg = threadIdx.x / kTC;  // 0..15
+  const uint32_t col = blockIdx.x * kTC + c;
   uint32_t w2[15];
 #pragma unroll
   for (int s = 4, i = 0; s < 8; s++)
@@ -440,10 +451,10 @@ __device__ __forceinline__ void fwd_cols_body(const NttArgs &a, const Limb &lb,
   }
   T *xt = reinterpret_cast<T *>(xch);
 #pragma unroll
-  for (int k = 0; k < 16; k++) xt[(rg + 16 * k) * kTileCols + c] = x[k];
+  for (int k = 0; k < 16; k++) xt[(rg + 16 * k) * kTC + c] = x[k];
   __syncthreads();
 #pragma unroll
-  for (int k = 0; k < 16; k++) x[k] = xt[(16 * rg + k) * kTileCols + c];
+  for (int k = 0; k < 16; k++) x[k] = xt[(16 * rg + k) * kTC + c];
   // stages 4..7: rows 16 rg + k
 #pragma unroll
   for (int s = 4, i = 0; s < 8; s++) {
@@ -460,9 +471,9 @@ __device__ __forceinline__ void fwd_cols_body(const NttArgs &a, const Limb &lb,
     st_nt<T>(dst, ((16 * rg + k) * kCols + col) * 4u, x[k]);
 }
 
-template <bool kPre>
-__global__ __launch_bounds__(512) void ntt_fwd_cols(NttArgs a) {
-  __shared__ int32_t xch[kRows * kTileCols];
+template <bool kPre, int kTC>
+__global__ __launch_bounds__(16 * kTC) void ntt_fwd_cols(NttArgs a) {
+  __shared__ int32_t xch[kRows * kTC];
   LimbMap m = a.map;
   if (a.group_alpha > 0) {
     const int g = a.group_period > 0 ? static_cast<int>(blockIdx.z) % a.group_period
@@ -479,8 +490,8 @@ __global__ __launch_bounds__(512) void ntt_fwd_cols(NttArgs a) {
   const void *src = sbase + (static_cast<size_t>(lb.sl) << kLogN);
   void *dst =
       poly_dst(a, blockIdx.z) + (static_cast<size_t>(lb.l) << kLogN);
-  const uint32_t col = blockIdx.x * kTileCols + (threadIdx.x & (kTileCols - 1));
-  const int rg = threadIdx.x / kTileCols;
+  const uint32_t col = blockIdx.x * kTC + (threadIdx.x & (kTC - 1));
+  const int rg = threadIdx.x / kTC;
   uint32_t x[16];
 #pragma unroll
   for (int k = 0; k < 16; k++)
@@ -488,9 +499,9 @@ __global__ __launch_bounds__(512) void ntt_fwd_cols(NttArgs a) {
   const uint32_t q = a.tab.q[lb.ti];
   const uint32_t qinv = static_cast<uint32_t>(a.tab.qinv[lb.ti]);
   if (q < (1u << 30))
-    fwd_cols_body<kPre, true>(a, lb, x, q, qinv, dst, xch);
+    fwd_cols_body<kPre, true, kTC>(a, lb, x, q, qinv, dst, xch);
   else
-    fwd_cols_body<kPre, false>(a, lb, x, q, qinv, dst, xch);
+    fwd_cols_body<kPre, false, kTC>(a, lb, x, q, qinv, dst, xch);
 }
 
 // forward, row pass: stages 8..15 (in place on dst) + epilogue
@@ -822,7 +833,7 @@ __global__ __launch_bounds__(256) void ntt_inv_rows(NttArgs a) {
 
 // inverse, column pass: GS stages 7..0 (in place on dst) + constant epilogue
 // (INTTPhase2 with MultConst / MultConstNormalize, NTTUtils.cuh:369-391)
-template <int kEpi, bool kLazy>
+template <int kEpi, bool kLazy, int kTC>
 __device__ __forceinline__ void inv_cols_body(const NttArgs &a, const Limb &lb,
                                               uint32_t (&xin)[16], uint32_t q,
                                               uint32_t qinv, uint32_t *dst,
@@ -831,9 +842,9 @@ __device__ __forceinline__ void inv_cols_body(const NttArgs &a, const Limb &lb,
   using T = typename A::T;
   const A ar(q, qinv);
   const uint32_t *tw = a.tab.itw + (static_cast<size_t>(lb.ti) << kLogN);
-  const int c = threadIdx.x & (kTileCols - 1);
-  const int rg = threadIdx.x / kTileCols;
-  const uint32_t col = blockIdx.x * kTileCols + c;
+  const int c = threadIdx.x & (kTC - 1);
+  const int rg = threadIdx.x / kTC;
+  const uint32_t col = blockIdx.x * kTC + c;
   uint32_t w2[15], w1[15];
 #pragma unroll
   for (int s = 4, i = 0; s < 8; s++)
@@ -861,10 +872,10 @@ __device__ __forceinline__ void inv_cols_body(const NttArgs &a, const Limb &lb,
   }
   T *xt = reinterpret_cast<T *>(xch);
 #pragma unroll
-  for (int k = 0; k < 16; k++) xt[(16 * rg + k) * kTileCols + c] = x[k];
+  for (int k = 0; k < 16; k++) xt[(16 * rg + k) * kTC + c] = x[k];
   __syncthreads();
 #pragma unroll
-  for (int k = 0; k < 16; k++) x[k] = xt[(rg + 16 * k) * kTileCols + c];
+  for (int k = 0; k < 16; k++) x[k] = xt[(rg + 16 * k) * kTC + c];
 #pragma unroll
   for (int s = 3; s >= 0; s--) {
     const int h = 8 >> s;
@@ -887,14 +898,14 @@ __device__ __forceinline__ void inv_cols_body(const NttArgs &a, const Limb &lb,
   }
 }
 
-template <int kEpi>
-__global__ __launch_bounds__(512) void ntt_inv_cols(NttArgs a) {
-  __shared__ int32_t xch[kRows * kTileCols];
+template <int kEpi, int kTC>
+__global__ __launch_bounds__(16 * kTC) void ntt_inv_cols(NttArgs a) {
+  __shared__ int32_t xch[kRows * kTC];
   const Limb lb = decode(a.map, blockIdx.y);
   uint32_t *dst =
       poly_dst(a, blockIdx.z) + (static_cast<size_t>(lb.l) << kLogN);
-  const uint32_t col = blockIdx.x * kTileCols + (threadIdx.x & (kTileCols - 1));
-  const int rg = threadIdx.x / kTileCols;
+  const uint32_t col = blockIdx.x * kTC + (threadIdx.x & (kTC - 1));
+  const int rg = threadIdx.x / kTC;
   uint32_t x[16];
 #pragma unroll
   for (int k = 0; k < 16; k++)
@@ -902,9 +913,9 @@ __global__ __launch_bounds__(512) void ntt_inv_cols(NttArgs a) {
   const uint32_t q = a.tab.q[lb.ti];
   const uint32_t qinv = static_cast<uint32_t>(a.tab.qinv[lb.ti]);
   if (q < (1u << 30))
-    inv_cols_body<kEpi, true>(a, lb, x, q, qinv, dst, xch);
+    inv_cols_body<kEpi, true, kTC>(a, lb, x, q, qinv, dst, xch);
   else
-    inv_cols_body<kEpi, false>(a, lb, x, q, qinv, dst, xch);
+    inv_cols_body<kEpi, false, kTC>(a, lb, x, q, qinv, dst, xch);
 }
 
 
@@ -1886,13 +1897,32 @@ __global__ __launch_bounds__(1024) void ntt_inv_1p(NttArgs a, int num_limbs,
     inv_1p_body<kEpi, false>(a, lb, z, s, q, qinv, lds);
 }
 
+template <int kTC>
+void launch_fwd_cols(const NttArgs &a, int num_limbs, int num_z,
+                     bool pre_const, hipStream_t s) {
+  const dim3 g(kCols / kTC, num_limbs, num_z), b(16 * kTC);
+  if (pre_const)
+    hipLaunchKernelGGL((ntt_fwd_cols<true, kTC>), g, b, 0, s, a);
+  else
+    hipLaunchKernelGGL((ntt_fwd_cols<false, kTC>), g, b, 0, s, a);
+}
+
+template <int kTC>
+void launch_inv_cols(const NttArgs &a, int num_limbs, int num_polys,
+                     int epilogue, hipStream_t s) {
+  const dim3 g(kCols / kTC, num_limbs, num_polys), b(16 * kTC);
+  if (epilogue == kEpiConstCentre)
+    hipLaunchKernelGGL((ntt_inv_cols<kEpiConstCentre, kTC>), g, b, 0, s, a);
+  else
+    hipLaunchKernelGGL((ntt_inv_cols<kEpiConst, kTC>), g, b, 0, s, a);
+}
+
 }  // namespace
 
 hipError_t launch_ntt_fwd_cols(const NttArgs &a, int num_limbs, int num_z,
                                hipStream_t s) {
   if (num_limbs <= 0 || num_z <= 0) return hipSuccess;
-  dim3 gc(kCols / kTileCols, num_limbs, num_z);
-  hipLaunchKernelGGL(ntt_fwd_cols<false>, gc, dim3(512), 0, s, a);
+  launch_fwd_cols<kTileCols>(a, num_limbs, num_z, false, s);
   return hipGetLastError();
 }
 
@@ -1928,14 +1958,19 @@ static uint32_t item_rcp(int num_limbs) {
 hipError_t launch_ntt_fwd(const NttArgs &a, int num_limbs, int num_polys,
                           bool pre_const, int epilogue, hipStream_t s) {
   if (num_limbs <= 0 || num_polys <= 0) return hipSuccess;
-  // The single pass takes one workgroup's latency however few limbs there
-  // are (12.3 us for 1 limb, 13.9 for 16, 16-17 for 64); up to 16 limbs
-  // the two passes, spread over many small workgroups, are faster (9.3 us
-  // for 1 limb, 11.3-12.5 for 2-16; from 24 limbs on they are not). The
-  // ModDown epilogue keeps the single pass: its caller makes that choice.
+  // The single pass runs in rounds of 64 limbs (four workgroups each, one
+  // per CU) and takes a whole round's time however full the last one is: 13.7
+  // us for 24 limbs, 13.9 for 32, 14.1 for 40, 14.7 for 64, 24.1 for 80,
+  // 24.7 for 96 (31-bit primes 15.8, 16.0, 16.2, 16.8, 27.1, 27.5). The two
+  // passes, spread over small workgroups, grow with the limbs: 11.6, 12.1,
+  // 14.6, 17.9, 23.7, 26.0 (12.3, 12.9, 15.7, 18.1, 23.1, 25.5). So two passes
+  // up to half a round and up to a quarter of the second; later rounds hide
+  // it (144 limbs 35.5 against 38.0 us). The ModDown epilogue keeps the
+  // single pass: its caller makes that choice.
   const int items = num_limbs * num_polys;
+  const bool one_pass = items > 32 && (items <= 64 || items > 80);
   if (a.src_disjoint && !a.fwd_two_pass &&
-      (epilogue == kEpiModDown || items > 16)) {
+      (epilogue == kEpiModDown || one_pass)) {
     dim3 g1(4 * ((items + 7) / 8 * 8));
     if (epilogue == kEpiModDown && a.src_bcast)
       hipLaunchKernelGGL(ntt_fwd_1p_bcast, g1, dim3(1024), 0, s, a,
@@ -1951,11 +1986,10 @@ hipError_t launch_ntt_fwd(const NttArgs &a, int num_limbs, int num_polys,
                          a, num_limbs, items, item_rcp(num_limbs));
     return hipGetLastError();
   }
-  dim3 gc(kCols / kTileCols, num_limbs, num_polys);
-  if (pre_const)
-    hipLaunchKernelGGL(ntt_fwd_cols<true>, gc, dim3(512), 0, s, a);
+  if (items <= kNarrowFwd)
+    launch_fwd_cols<kNarrowCols>(a, num_limbs, num_polys, pre_const, s);
   else
-    hipLaunchKernelGGL(ntt_fwd_cols<false>, gc, dim3(512), 0, s, a);
+    launch_fwd_cols<kTileCols>(a, num_limbs, num_polys, pre_const, s);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   return launch_ntt_fwd_rows(a, num_limbs, num_polys, epilogue, s);
@@ -1963,11 +1997,10 @@ hipError_t launch_ntt_fwd(const NttArgs &a, int num_limbs, int num_polys,
 
 hipError_t launch_ntt_inv_cols(const NttArgs &a, int num_limbs, int num_polys,
                                int epilogue, hipStream_t s) {
-  dim3 gc(kCols / kTileCols, num_limbs, num_polys);
-  if (epilogue == kEpiConstCentre)
-    hipLaunchKernelGGL(ntt_inv_cols<kEpiConstCentre>, gc, dim3(512), 0, s, a);
+  if (num_limbs * num_polys <= kNarrowInv)
+    launch_inv_cols<kNarrowCols>(a, num_limbs, num_polys, epilogue, s);
   else
-    hipLaunchKernelGGL(ntt_inv_cols<kEpiConst>, gc, dim3(512), 0, s, a);
+    launch_inv_cols<kTileCols>(a, num_limbs, num_polys, epilogue, s);
   return hipGetLastError();
 }
 

@@ -21,7 +21,8 @@ def chd():
 
 
 @pytest.mark.parametrize("limbs,polys", [
-    (1, 1), (12, 1), (13, 1), (4, 4), (17, 1), (16, 2), (33, 1), (13, 5)])
+    (1, 1), (12, 1), (13, 1), (4, 4), (17, 1), (16, 2), (33, 1), (13, 5),
+    (27, 3)])
 def test_ntt_mixed_primes(chd, limbs, polys):
     primes = [(Q31 if i % 2 == 0 else Q30)[i // 2] for i in range(limbs)]
     plan = chd.NttPlan(primes)
