@@ -43,8 +43,10 @@ BCONV_TRAFFIC = 12741632
 # config 4 HMult compulsory bytes: 4 x 24 input limbs, 3 x 2 x 32 key limbs,
 # 2 x 23 output limbs
 HMULT_BYTES = (96 + 192 + 46) * 4 * (1 << 16)
-# its measured HBM bytes per HMult, the sum over its 8 launches
-# (profiles/hmult_config4_traffic.md, one row per launch)
+# its measured HBM bytes per HMult, the sum over its 5 launches
+# (profiles/hmult_switch_config4_traffic.md, one row per launch)
+HMULT_SWITCH_TRAFFIC = 27440128 + 26079232 + 134737536 + 17345536 + 44419072
+# and of the eight-launch form before it (profiles/hmult_config4_traffic.md)
 HMULT_TRAFFIC = (25288704 + 12904384 + 25421824 + 38169344 + 128323392 +
                  9696448 + 16902144 + 48662528)
 N = 1 << 16
@@ -681,17 +683,18 @@ def main():
                      "frac": bconv_tops / INT8_PEAK_TOPS},
         },
         "roofline_hmult": {
-            "kernel": "HMult key switch + merged rescale, config 4 (8 "
+            "kernel": "HMult key switch + merged rescale, config 4 (5 "
                       "launches), inputs and key cold",
             "bound": "hbm",
             "achieved": hmult_gbs,
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": hmult_gbs / HBM_PEAK_GBS,
-            "traffic": HMULT_TRAFFIC,
+            "traffic": HMULT_SWITCH_TRAFFIC,
             "note": "achieved = compulsory %d B (96 limbs in, 192 key limbs, "
-                    "46 limbs out) / HMult time; traffic = the 8 launches' "
-                    "counted HBM bytes" % HMULT_BYTES,
+                    "46 limbs out) / HMult time; traffic = the 5 launches' "
+                    "counted HBM bytes (%d B as eight launches)"
+                    % (HMULT_BYTES, HMULT_TRAFFIC),
         },
         "extra": {
             "ntt_forward_us": fwd_ms * 1e3,

@@ -78,3 +78,20 @@ def test_hmult_launch_count_matches_trace():
              re.finditer(r"\| `([^`]+)` \| (\d+) \|", text)}
     steps = calls["modup_keyacc"]
     assert sum(calls.values()) == 8 * steps
+
+
+def test_hmult_switch_traffic_matches_profile():
+    """the bench's HMult traffic is the sum of the profile's five per-launch
+    rows, each consistent with its counters"""
+    rows = []
+    with open(os.path.join(ROOT, "profiles",
+                           "hmult_switch_config4_traffic.md")) as f:
+        for line in f:
+            cells = [c.strip() for c in line.strip().strip("|").split("|")]
+            if len(cells) == 8 and cells[0].isdigit():
+                rows.append(cells)
+    assert [int(c[0]) for c in rows] == list(range(1, 6))
+    for c in rows:
+        fetch, write, total = float(c[3]), float(c[4]), int(c[7])
+        assert abs(total - (fetch * 2 + write) * 1024) < 1024
+    assert bench.HMULT_SWITCH_TRAFFIC == sum(int(c[7]) for c in rows)
