@@ -332,7 +332,8 @@ __device__ __forceinline__ u32x4 blocked_lds4(const uint32_t *xt, int v) {
 
 // Per-limb arithmetic policy. Values between the two passes of a transform
 // stay unreduced in the policy's range: [0, 4q) (forward) and [0, 2q)
-// (inverse) for q < 2^30, [0, 2q) and [0, q) for q < 2^31.
+// (inverse) for q < 2^30, [0, 2q) and [0, q) for q < 2^31. A transform of a
+// prime of the second kind takes signed representatives in [-q, q) too.
 template <bool kLazy>
 struct Arith;
 
@@ -430,7 +431,8 @@ __device__ __forceinline__ void fwd_cols_body(const NttArgs &a, const Limb &lb,
 
   T x[16];
 #pragma unroll
-  for (int k = 0; k < 16; k++) x[k] = static_cast<T>(xin[k]);
+  for (int k = 0; k < 16; k++)
+    x[k] = kLazy ? xin[k] : umin(xin[k], xin[k] + q);  // [-q, q) to [0, q)
   if constexpr (kPre) {
     const uint32_t ce = a.cst[lb.ci];
     const uint32_t ceq = ar.twq(ce);
@@ -827,8 +829,11 @@ __global__ __launch_bounds__(256) void ntt_inv_rows(NttArgs a) {
   for (int k = 0; k < 16; k++) x[k] = xr[pidx(16 * c + k)];
   if (q < (1u << 30))
     inv_rows_body<true>(w1, w2, x, q, qinv, dst, xch, kBlocked);
-  else
+  else {
+#pragma unroll
+    for (int k = 0; k < 16; k++) x[k] = umin(x[k], x[k] + q);  // from [-q, q)
     inv_rows_body<false>(w1, w2, x, q, qinv, dst, xch, kBlocked);
+  }
 }
 
 // inverse, column pass: GS stages 7..0 (in place on dst) + constant epilogue
@@ -1413,8 +1418,9 @@ __device__ __forceinline__ void fwd_1p_body(const NttArgs &a, const Limb &lb,
   // registers of the 64 both have. In the lazy body this barrier costs 1.2 us.
   if constexpr (!kLazy) __builtin_amdgcn_sched_barrier(0);
   // ---- round 1: stages 0, 1 of quarter j (bits 15, 14), then 2..5.
-  // Stages 0 and 1 are one 64-bit dot product and one reduction per output
-  // (canonical inputs and constants: below 4 q^2 < 2^64).
+  // Stages 0 and 1 are one 64-bit dot product and one reduction per output:
+  // canonical inputs and constants below q 2^32 for q < 2^30; above, inputs
+  // in [-q, q) and centred constants, below 2 q^2 < 2^63 in size.
   {
     const uint32_t qn = ar.qn;
     const uint32_t w01 = mont_mad(w0, w1, w1 * qn, q);
@@ -1435,6 +1441,10 @@ __device__ __forceinline__ void fwd_1p_body(const NttArgs &a, const Limb &lb,
         c[i] = umin(v, v - q);
       }
     }
+    if constexpr (!kLazy) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) c[i] = c[i] > (q >> 1) ? c[i] - q : c[i];
+    }
 #pragma unroll
     for (int k = 0; k < 16; k++) {
       const uint32_t so = 4u * static_cast<uint32_t>(k << 10);
@@ -1443,12 +1453,12 @@ __device__ __forceinline__ void fwd_1p_body(const NttArgs &a, const Limb &lb,
       const uint32_t x2 = bld1<kSrcAux>(rsrc, vt, so + 8u * kQuarter);
       const uint32_t x3 = bld1<kSrcAux>(rsrc, vt, so + 12u * kQuarter);
       uint64_t acc;
-      if constexpr (kBcast) {
-        // centred inputs of a source prime below 2^31, |x| < 2^30, times
-        // constants below q: the signed sum lies in (-q 2^32, q 2^32);
-        // adding q 2^32 (= 0 mod q) makes it positive and below q 2^33 <
-        // 2^64
-        acc = (static_cast<uint64_t>(q) << 32) +
+      if constexpr (kBcast || !kLazy) {
+        // signed inputs. Lazy form: centred ones of a source prime below
+        // 2^31, |x| < 2^30, times constants below q, so the sum lies in
+        // (-q 2^32, q 2^32); adding q 2^32 (= 0 mod q) makes it positive
+        // and below q 2^33 < 2^63
+        acc = (kLazy ? static_cast<uint64_t>(q) << 32 : 0) +
               static_cast<uint64_t>(
                   static_cast<int64_t>(static_cast<int32_t>(x0)) *
                       static_cast<int32_t>(c[0]) +
@@ -1471,11 +1481,10 @@ __device__ __forceinline__ void fwd_1p_body(const NttArgs &a, const Limb &lb,
         x[k] =
             static_cast<uint32_t>((static_cast<uint64_t>(m) * q + acc) >> 32);
       } else {
-        // the high word, below 2q, is reduced on its own: the 64-bit sum of
-        // both could overflow. [0, q) + [0, q] is below 2q for the words
-        // that occur (reduce_sum4)
+        // the high word, in [-q, q), is reduced on its own: [0, q) plus the
+        // low word's reduction in [0, q] is below 2q
         const uint32_t hi = static_cast<uint32_t>(acc >> 32);
-        x[k] = umin(hi, hi - q) +
+        x[k] = umin(hi, hi + q) +
                static_cast<uint32_t>((static_cast<uint64_t>(m) * q +
                                       static_cast<uint32_t>(acc)) >>
                                      32);

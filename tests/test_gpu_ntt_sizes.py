@@ -58,3 +58,30 @@ def test_ntt_mixed_primes(chd, limbs, polys):
         z = dev(x)
         plan.inverse(z, z, limbs, polys, mont_conv=mont)
         assert np.array_equal(host(z), want)
+
+
+@pytest.mark.parametrize("limbs", [3, 40])
+def test_ntt_signed_representatives(chd, limbs):
+    """primes above 2^30 take any representative in [-q, q), to both ends of
+    it, in every form of the transform"""
+    primes = Q31[:limbs]
+    plan = chd.NttPlan(primes)
+    x = uniform_limbs(np.random.default_rng(0x519 + limbs), primes)
+    q = np.array(primes, np.int64)[:, None]
+    x[:, 0:512] = 0
+    x[:, 512:1024] = q - 1
+    low = np.arange(N) % 3 == 0
+    low[256:768] = True
+    y = (x.astype(np.int64) - np.where(low, q, 0)).astype(np.int32)
+    assert y.min() == -max(primes)
+    src, out = dev(y.view(np.uint32)), zeros(limbs, N)
+    flat = np.ascontiguousarray(x).reshape(-1)
+    for mont in (False, True):
+        want = _orc.ntt_batch(flat, 16, primes, int(mont)).reshape(limbs, N)
+        for kw in ({}, {"two_pass": True}):
+            plan.forward(out, src, limbs, mont_conv=mont, **kw)
+            assert np.array_equal(host(out), want), kw
+        want = _orc.intt_batch(flat, 16, primes, int(mont)).reshape(limbs, N)
+        for kw in ({}, {"single_pass": True}):
+            plan.inverse(out, src, limbs, mont_conv=mont, **kw)
+            assert np.array_equal(host(out), want), kw
