@@ -333,9 +333,9 @@ __global__ __launch_bounds__(kThreads) void bs_fused_kernel(chd_tables t,
   }
 }
 
-// r += t 2^-32 mod q for a sum t of four products of canonical residues.
-// kSmall (q < 2^30): t < q 2^32, so one Montgomery reduction is in [0, 2q),
-// where r stays too; otherwise r is canonical.
+// r += t 2^-32 mod q. kSmall (q < 2^30): t < q 2^32 (a sum of four products of
+// canonical residues), so one Montgomery reduction is in [0, 2q), where r
+// stays too; otherwise t < 4 q^2 and r is canonical.
 template <bool kSmall>
 __device__ __forceinline__ void gs_acc(uint32_t &r, uint64_t t, uint32_t q,
                                        uint32_t qn) {
@@ -358,17 +358,24 @@ __device__ __forceinline__ void gs_acc(uint32_t &r, uint64_t t, uint32_t q,
 // loads are all issued before the products: an absent plaintext (or a baby
 // step past the last) reads the baby step's words instead and counts as zero,
 // where a branch around each load had it wait for the one before. One giant
-// step has a single plaintext per baby step and takes them one by one, with
-// default loads. Giant x baby steps on 13 + 8 limbs: 1 x 8 24.0 -> 22.0 us,
-// 2 x 8 37.1 -> 34.8, 4 x 8 66.6 -> 54.0 (5.5 TB/s), 6 x 6 78 -> 60, 8 x 8 131
-// -> 93. Baby steps in fours: 57.8 us at 4 x 8 (5 instead of 7 waves per SIMD)
-// and 25.8 at 1 x 8.
+// step has a single plaintext per baby step and takes them one by one with
+// default loads, absent ones left out (masked, each plaintext was waited for
+// before the baby step's loads: 47 instead of 43 us at 1 x 16). Giant x baby
+// steps on 13 + 8 limbs: 1 x 8 24.0 -> 22.0 us, 2 x 8 37.1 -> 34.8, 4 x 8 66.6
+// -> 54.0 (5.5 TB/s), 6 x 6 78 -> 60, 8 x 8 131 -> 93. Baby steps in fours:
+// 57.8 us at 4 x 8 (5 instead of 7 waves per SIMD) and 25.8 at 1 x 8.
+// Plaintext and baby-step words are signed representatives in (-q, q): the two
+// products of a pair lie in (-2 q^2, 2 q^2), and their sum starts at a multiple
+// of q that makes it positive and keeps it in gs_acc's range (q 2^31 >= 2 q^2
+// for q < 2^30, otherwise 2 q^2), which the multiply-add takes for free.
 template <int kG, bool kSmall>
 __device__ __forceinline__ void gs_fused_body(const chd_gs_args &a,
                                               const LimbIdx &li) {
   constexpr int kU = kG == 1 ? 1 : 2;
   const uint32_t q = li.q;
   const uint32_t qn = 0u - static_cast<uint32_t>(li.qinv);
+  const uint64_t bias = kSmall ? static_cast<uint64_t>(q) << 31
+                               : 2 * static_cast<uint64_t>(q) * q;
   const size_t o = (static_cast<size_t>(li.l) << kLogN) +
                    blockIdx.x * kCoefPerBlock + threadIdx.x * kPerThread;
   uint32_t rb[kG][4], ra[kG][4];
@@ -387,6 +394,7 @@ __device__ __forceinline__ void gs_fused_body(const chd_gs_args &a,
     }
   }
   for (int b0 = 0; b0 < a.num_bs; b0 += kU) {
+    if (kG == 1 && a.pt[0][b0] == nullptr) continue;
     uint4 xb[kU], xa[kU];
 #pragma unroll
     for (int j = 0; j < kU; j++) {
@@ -403,18 +411,19 @@ __device__ __forceinline__ void gs_fused_body(const chd_gs_args &a,
       for (int j = 0; j < kU; j++) {
         const int b = min(b0 + j, a.num_bs - 1);
         const uint32_t *pt = a.pt[g][b];
-        mask[j] = pt != nullptr && b0 + j < a.num_bs ? ~0u : 0u;
-        const uint32_t *p = (pt != nullptr ? pt : a.bs_b[b]) + o;
+        const bool real = kG == 1 || pt != nullptr;
+        mask[j] = real && b0 + j < a.num_bs ? ~0u : 0u;
+        const uint32_t *p = (real ? pt : a.bs_b[b]) + o;
         mv[j] = kG == 1 ? ld4(p) : ld4_once(p);
       }
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        uint64_t tb = 0, ta = 0;
+        uint64_t tb = bias, ta = bias;
 #pragma unroll
         for (int j = 0; j < kU; j++) {
-          const uint64_t mm = get(mv[j], i) & mask[j];
-          tb += mm * get(xb[j], i);
-          ta += mm * get(xa[j], i);
+          const int64_t mm = static_cast<int32_t>(get(mv[j], i) & mask[j]);
+          tb += static_cast<uint64_t>(mm * static_cast<int32_t>(get(xb[j], i)));
+          ta += static_cast<uint64_t>(mm * static_cast<int32_t>(get(xa[j], i)));
         }
         gs_acc<kSmall>(rb[g][i], tb, q, qn);
         gs_acc<kSmall>(ra[g][i], ta, q, qn);

@@ -357,7 +357,8 @@ int chd_k_zero(uint32_t *dst, long long words, void *stream);
  * src/extension/Hoist.cu:80-118, 334-445): for every giant step g of the
  * launch, dst_g = [dst_g +] sum_b MontMul(pt[g][b], bs_b) for both parts,
  * over num_limbs extended-basis limbs. Each baby step is read once per
- * launch. pt[g][b] NULL skips the pair. */
+ * launch. pt[g][b] NULL skips the pair. Plaintext and baby-step words may be
+ * any representatives in (-q, q), as signed integers. */
 #define CHD_GS_MAX_BS 32
 #define CHD_GS_MAX_GS 8
 typedef struct chd_gs_args {
