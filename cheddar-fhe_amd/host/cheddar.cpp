@@ -23,6 +23,24 @@ void K(int status) {
 
 int DivCeil(int a, int b) { return (a + b - 1) / b; }
 
+// Rescale's destination limbs (of all polynomials) above which the single
+// pass that forms the one-source BConv itself takes over from the column
+// stage: it runs in rounds of 64 limbs and takes a round's time however full
+// the round is, where the column stage, with half of the chip per polynomial,
+// grows with the limbs. Microseconds, column stage / single pass, at 16, 24,
+// 28, 32, 40 limbs of one polynomial: 23.1, 26.6, 28.4, 29.8, 34.0 / 27.0,
+// 27.3, 27.4, 27.5, 27.4; at 24, 32, 34, 48, 64, 66, 80 of two: 25.2, 26.6,
+// 29.0, 31.9, 37.6, 41.4, 42.1 / 27.6, 27.3, 27.2, 27.7, 28.3, 38.2, 39.2.
+// With destinations above 2^30 the single pass takes longer: 23.9, 28.2, 30.9,
+// 31.9, 36.3 / 31.9, 32.4, 32.5, 32.5, 32.7 and at 32, 44, 48, 64, 68, 80, 84:
+// 27.6, 32.6, 33.4, 39.9, 43.5, 44.3, 47.3 / 33.0, 32.7, 32.8, 33.3, 45.9,
+// 46.8, 47.0.
+bool SinglePassRescale(int num_polys, int dst_len, bool wide_primes) {
+  const int limbs = num_polys * dst_len;
+  if (!wide_primes) return limbs > (num_polys == 1 ? 24 : 32);
+  return limbs > (num_polys == 1 ? 32 : 44) && (limbs <= 64 || limbs > 80);
+}
+
 // 1: a hoisting handle with a wide giant-step accumulation keeps a tiled
 // copy of its plaintexts beside the per-pair ones (twice their memory); 0:
 // the accumulation reads the per-pair plaintexts in place
@@ -847,6 +865,8 @@ void ModSwitchHandler<uint32_t>::BuildSwitch(
                           restore_lo, restore_hi, &c1, &c2);
   st.src_len = sl;
   st.dst_len = dl;
+  st.wide = std::any_of(dst.begin(), dst.end(),
+                        [](word p) { return p >= (1u << 30); });
   st.const1.resize(sl);
   HipCheck(hipMemcpy(st.const1.data(), c1.data(), sl * sizeof(word),
                      hipMemcpyHostToDevice),
@@ -856,6 +876,16 @@ void ModSwitchHandler<uint32_t>::BuildSwitch(
   K(chd_bconv_table_pack(packed.data(), c2.data(), dst.data(), sl, dl));
   st.table.Resize(packed.size());
   st.table.Upload(packed.data(), packed.size());
+  if (sl == 1) {
+    std::vector<word> col(dl);
+    for (int k = 0; k < dl; k++)
+      col[k] = c2[k] < 0 ? static_cast<word>(c2[k] + static_cast<int64_t>(dst[k]))
+                         : static_cast<word>(c2[k]);
+    st.bconv1.resize(dl);
+    HipCheck(hipMemcpy(st.bconv1.data(), col.data(), dl * sizeof(word),
+                       hipMemcpyHostToDevice),
+             "hipMemcpy");
+  }
 }
 
 // src/core/ModSwitch.cu:429-509 up to the forward row pass: the inverse row
@@ -1094,9 +1124,8 @@ void ModSwitchHandler<uint32_t>::ModDownMulti(const std::vector<word *> &dst,
                "ModDown: src and dst should be different");
   }
   // NTTForModDown's epilogue operand src2 (the kept limbs of the source) is
-  // read while other workgroups write the destinations, and with few
-  // destination limbs the BConv writes them before that: no destination
-  // may overlap any polynomial's src2, checked before anything is launched
+  // read while other workgroups write the destinations: no destination may
+  // overlap any polynomial's src2, checked before anything is launched
   const int src2_off = std::max(0, np_src.num_ter_ - np_dst.num_ter_);
   const int s2_lo = np_dst.num_ter_ - np_non_intt.num_ter_;
   const int s2_hi = s2_lo + np_non_intt.GetNumQ();
@@ -1128,12 +1157,6 @@ void ModSwitchHandler<uint32_t>::ModDownMulti(const std::vector<word *> &dst,
     mi.tab_gap = param_.GetMaxNumMain() + np_non_intt.num_ter_;
     mi.src_gap = np_src.GetNumQ() - mi.num_q;
   }
-  if (intt_rows != nullptr)
-    // the first pass was done by the key accumulation (ModDownInttRange)
-    AssertTrue(!intt_on_ter, "ModDown: fused INTT needs main INTT limbs");
-  else
-    K(chd_k_ntt_inv_rows(&ntt_.Tables(), &mi, intt, ilen, src + off, nullptr,
-                         src_pstride, src_len, num_polys, CurrentStream()));
   chd_limb_map m = NoSkipMap(param_, np_dst);
   const DeviceVector<word> &ipp =
       kind == Kind::ModDown   ? inv_prime_prod_
@@ -1147,9 +1170,29 @@ void ModSwitchHandler<uint32_t>::ModDownMulti(const std::vector<word *> &dst,
                                        : mod_down_rescale_padding_;
   const word *pad =
       kind != Kind::ModDown && padv.size() != 0 ? padv.data() : nullptr;
-  // the column stage, then the row pass with the epilogue (NTTForModDown,
-  // NTT.cu:417-604) whose src2 are the untouched low limbs (src2_off, s2_lo,
-  // s2_hi above)
+  if (src_len == 1 && intt_rows == nullptr && galois == 1 &&
+      SinglePassRescale(num_polys, dst_len, st.wide)) {
+    // the INTT of the source limb in its two passes, then a single pass that
+    // forms each destination's BConv, the source times that limb's table
+    // entry, as it reads it
+    K(chd_k_ntt_inv(&ntt_.Tables(), &mi, intt, ilen, src + off, src_pstride, 1,
+                    num_polys, st.const1.data(), 1, CurrentStream()));
+    K(chd_k_ntt_fwd_moddown_bconv1_multi(
+        &ntt_.Tables(), &m, dst.data(), num_polys, dst_len,
+        reinterpret_cast<const int32_t *>(intt), ilen, st.bconv1.data(),
+        src + static_cast<size_t>(src2_off) * n, src_pstride, s2_lo, s2_hi,
+        ipp.data(), pad, CurrentStream()));
+    return;
+  }
+  // the inverse row pass, the column stage, then the row pass with the
+  // epilogue (NTTForModDown, NTT.cu:417-604) whose src2 are the untouched low
+  // limbs (src2_off, s2_lo, s2_hi above)
+  if (intt_rows != nullptr)
+    // the first pass was done by the key accumulation (ModDownInttRange)
+    AssertTrue(!intt_on_ter, "ModDown: fused INTT needs main INTT limbs");
+  else
+    K(chd_k_ntt_inv_rows(&ntt_.Tables(), &mi, intt, ilen, src + off, nullptr,
+                         src_pstride, src_len, num_polys, CurrentStream()));
   Scratch conv(ws_, static_cast<size_t>(num_polys) * dst_len * n);
   const long long clen = static_cast<long long>(dst_len) * n;
   chd_switch_job jobs[CHD_MAX_JOBS] = {};

@@ -486,14 +486,9 @@ def test_hmult_in_place_and_separate_rescale(chd, ks):
 
 @pytest.mark.parametrize("rescale", [True, False])
 def test_hmult_one_aux_prime(chd, rescale):
-    """alpha = 1 (dnum = L = 4): ModDown has a single source limb. With so
-    few destination limbs (at most 12 polynomial-limbs for one source) the
-    one-source BConv writes the destination and the two-pass ModDown NTT
-    runs in place on it; without rescale the result is also rescaled
-    separately (one source again, the same path), both against the oracle.
-    The one-source BConv formed inside the single-pass NTT serves more
-    destination limbs and is pinned by the L = 24 Rescale tests and
-    test_rescale_either_side_of_the_one_source_limit."""
+    """alpha = 1 (dnum = L = 4): ModDown has a single source limb, whose
+    inverse row pass the key accumulation did; without rescale the result is
+    also rescaled separately (one source again), both against the oracle."""
     main, aux, L = Q30[:4], Q31[:1], 4
     param = chd.Param(main, aux, [(i, 0) for i in range(1, L + 1)])
     ctx = chd.Context(param)
@@ -515,14 +510,12 @@ def test_hmult_one_aux_prime(chd, rescale):
         assert np.array_equal(host(out[1]), _orc.rescale(wa, main, L, 1, 16))
 
 
-@pytest.mark.parametrize("L", [7, 8, 13, 14])
+@pytest.mark.parametrize("L", [7, 8, 13, 14, 17, 18])
 def test_rescale_either_side_of_the_one_source_limit(chd, ks, L):
-    """Rescale has one source limb: up to 12 destination polynomial-limbs
-    the BConv writes the destination and a two-pass NTT runs in place on
-    it, above that the single-pass NTT forms the BConv as it reads. The
-    ciphertext (2 x 6 = 12 limbs at L = 7, 2 x 7 = 14 at L = 8) and the
-    single polynomial (12 at L = 13, 13 at L = 14) on both sides, against
-    the oracle"""
+    """Rescale has one source limb: up to 32 destination limbs of two
+    polynomials run the column stage, above that the single-pass NTT forms the
+    BConv as it reads. The ciphertext (2 x 16 limbs at L = 17, 2 x 17 at
+    L = 18) on both sides and the single polynomial, against the oracle"""
     param, ctx, main, aux = ks
     r = rng(490 + L)
     b, a = uniform_limbs(r, main[:L]), uniform_limbs(r, main[:L])
@@ -538,9 +531,8 @@ def test_rescale_either_side_of_the_one_source_limit(chd, ks, L):
 @pytest.mark.parametrize("L", [4, 24])
 def test_rescale_rejects_result_overlapping_kept_limbs(chd, ks, L):
     """a Rescale whose result bx is the input's ax overlaps the kept source
-    limbs the ModDown epilogue reads: the call fails before any launch
-    (also where few destination limbs let the BConv write the destination
-    first) and the input is left as it was"""
+    limbs the ModDown epilogue reads: the call fails before any launch and
+    the input is left as it was"""
     param, ctx, main, aux = ks
     r = rng(480 + L)
     b, a = uniform_limbs(r, main[:L]), uniform_limbs(r, main[:L])

@@ -64,6 +64,35 @@ def test_base_switch_shapes(chd, L, alpha, mixed):
     assert np.array_equal(host(out), _orc.mod_down(xq, main, L - 1, 16))
 
 
+@pytest.mark.parametrize("wide,L", [
+    (False, 17), (False, 18), (False, 25), (False, 26), (True, 23),
+    (True, 24), (True, 33), (True, 34), (True, 41), (True, 42)])
+def test_rescale_around_the_single_pass_limits(chd, wide, L):
+    """Rescale of one polynomial and of two on both sides of the limb counts
+    where the single pass and the column stage take turns: 24 and 2 x 16
+    destinations below 2^30; 32, 2 x 22 and 2 x 32 to 2 x 40 with larger
+    ones"""
+    main = [p for pair in zip(Q30[:21], Q31[8:29]) for p in pair] if wide \
+        else Q30[:26]
+    main = main[:L]
+    ctx = chd.Context(chd.Param(main, Q31[:8], [(L - 1, 0), (L, 0)]))
+    r = np.random.default_rng(0x5E5C + 64 * wide + L)
+    q = np.array(main, np.uint32)[:, None]
+    x = [uniform_limbs(r, main) for _ in range(2)]
+    for y in x:
+        y[:, :256] = q - 1
+        y[:, 256:512] = 0
+        y[-1, 512:768] = q[-1] // 2 + np.arange(256) % 2  # either sign
+    want = [_orc.rescale(y, main, L, 1, 16) for y in x]
+    res = (zeros(L - 1, N), zeros(L - 1, N))
+    ctx.rescale(1, res, (dev(x[0]), dev(x[1])))
+    assert np.array_equal(host(res[0]), want[0])
+    assert np.array_equal(host(res[1]), want[1])
+    one = zeros(L - 1, N)
+    ctx.rescale_poly(1, one, dev(x[0]))
+    assert np.array_equal(host(one), want[0])
+
+
 @pytest.mark.parametrize("rot", [1, 2, 255, 256, 1 << 14, N // 2 - 1])
 def test_rotation_in_the_last_row_pass(chd, rot):
     """HRot, whose automorphism runs inside ModDown's last pass, for factors
