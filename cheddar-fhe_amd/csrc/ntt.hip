@@ -47,13 +47,16 @@ constexpr int kCols = 256;
 // columns (256 threads instead of 512) shorten: forward and back in two
 // passes each, 1 limb 8.5 + 8.3 -> 7.8 + 7.9 us, 8 limbs 9.5 + 9.1 -> 8.8 +
 // 8.7, 12 limbs 9.9 + 9.2 -> 9.5 + 9.2, 16 limbs 10.4 + 9.1 -> 10.0 + 9.8
-// (31-bit primes 11.4 + 10.4 -> 10.6 + 10.6). With more limbs the halved
-// pieces of a row cost bandwidth (24 limbs 11.5 + 10.5 against 12.8 + 12.5).
-// 8 and 4 columns are slower than 16 at every size.
+// (31-bit primes 11.4 + 10.4 -> 10.6 + 10.6), as time on the device: a caller
+// that enqueues one small call at a time sees its host time instead. With more
+// limbs the halved pieces of a row cost bandwidth (24 limbs 11.5 + 10.5
+// against 12.8 + 12.5), and sooner where the forward pass works in place (13
+// limbs 10.9 against 11.0, 16 limbs 11.3 against 11.6). 8 and 4 columns are
+// slower than 16 at every size.
 constexpr int kTileCols = 32;
 constexpr int kNarrowCols = 16;
-constexpr int kNarrowFwd = 16;  // limbs of all polynomials
-constexpr int kNarrowInv = 12;
+constexpr int kNarrowFwd = 16;      // limbs of all polynomials
+constexpr int kNarrowInPlace = 12;  // forward in place, and the inverse
 constexpr int kTileRows = 16;   // rows per row-pass workgroup
 constexpr int kRowPad = kCols + kCols / 16;
 
@@ -478,8 +481,11 @@ __global__ __launch_bounds__(16 * kTC) void ntt_fwd_cols(NttArgs a) {
   __shared__ int32_t xch[kRows * kTC];
   LimbMap m = a.map;
   if (a.group_alpha > 0) {
-    const int g = a.group_period > 0 ? static_cast<int>(blockIdx.z) % a.group_period
-                                     : static_cast<int>(blockIdx.z);
+    // the division's result is in a vector register, and the limb's indices
+    // of every launch would be too (0.1 us per pass)
+    const int g = uniform(a.group_period > 0
+                              ? static_cast<int>(blockIdx.z) % a.group_period
+                              : static_cast<int>(blockIdx.z));
     m.skip_lo = group_lo(g, a.group_alpha, a.group_shift);
     m.skip_len =
         group_hi(g, a.group_alpha, a.group_shift, m.num_q) - m.skip_lo;
@@ -622,8 +628,11 @@ __global__ __launch_bounds__(256) void ntt_fwd_rows(NttArgs a) {
   __shared__ int32_t xch[kTileRows * kRowPad];
   LimbMap m = a.map;
   if (a.group_alpha > 0) {
-    const int g = a.group_period > 0 ? static_cast<int>(blockIdx.z) % a.group_period
-                                     : static_cast<int>(blockIdx.z);
+    // the division's result is in a vector register, and the limb's indices
+    // of every launch would be too (0.1 us per pass)
+    const int g = uniform(a.group_period > 0
+                              ? static_cast<int>(blockIdx.z) % a.group_period
+                              : static_cast<int>(blockIdx.z));
     m.skip_lo = group_lo(g, a.group_alpha, a.group_shift);
     m.skip_len =
         group_hi(g, a.group_alpha, a.group_shift, m.num_q) - m.skip_lo;
@@ -1995,7 +2004,7 @@ hipError_t launch_ntt_fwd(const NttArgs &a, int num_limbs, int num_polys,
                          a, num_limbs, items, item_rcp(num_limbs));
     return hipGetLastError();
   }
-  if (items <= kNarrowFwd)
+  if (items <= (a.src_disjoint ? kNarrowFwd : kNarrowInPlace))
     launch_fwd_cols<kNarrowCols>(a, num_limbs, num_polys, pre_const, s);
   else
     launch_fwd_cols<kTileCols>(a, num_limbs, num_polys, pre_const, s);
@@ -2006,7 +2015,7 @@ hipError_t launch_ntt_fwd(const NttArgs &a, int num_limbs, int num_polys,
 
 hipError_t launch_ntt_inv_cols(const NttArgs &a, int num_limbs, int num_polys,
                                int epilogue, hipStream_t s) {
-  if (num_limbs * num_polys <= kNarrowInv)
+  if (num_limbs * num_polys <= kNarrowInPlace)
     launch_inv_cols<kNarrowCols>(a, num_limbs, num_polys, epilogue, s);
   else
     launch_inv_cols<kTileCols>(a, num_limbs, num_polys, epilogue, s);
