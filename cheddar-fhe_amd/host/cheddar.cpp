@@ -147,20 +147,20 @@ uint32_t *Workspace::Push(size_t words) {
 }
 
 // false where nothing may be allocated: the bound is reached, the memory is
-// not there, or the stream is being captured (a plain allocation would end
-// the capture)
+// not there, or the calling stream is being captured
 bool Workspace::AddChunk(size_t words) {
   const size_t bytes = words * sizeof(uint32_t);
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (bytes > kMaxExtraBytes - extra_bytes_ ||
-      hipStreamIsCapturing(CurrentStream(), &st) != hipSuccess ||
-      st != hipStreamCaptureStatusNone)
-    return false;
+  if (bytes > kMaxExtraBytes - extra_bytes_) return false;
+  const hipError_t e = hipStreamIsCapturing(CurrentStream(), &st);
+  if (e != hipSuccess) (void)hipGetLastError();  // not the next launch's
+  if (e != hipSuccess || st != hipStreamCaptureStatusNone) return false;
   Chunk c;
   try {
+    RelaxedCapture relaxed;
     c.buf.Resize(bytes);
   } catch (const std::exception &) {
-    (void)hipGetLastError();  // not the next launch's failure
+    (void)hipGetLastError();
     return false;
   }
   c.base = c.buf.as<uint32_t>();

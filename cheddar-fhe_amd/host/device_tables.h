@@ -16,6 +16,24 @@ namespace cheddar {
 // Throws with the HIP error text; C-ABI entry points catch and convert.
 void HipCheck(hipError_t e, const char *what);
 
+// While one lives, this thread's allocations leave a graph that another thread
+// records alone: in that thread's global capture mode they would fail and end
+// its recording.
+class RelaxedCapture {
+ public:
+  RelaxedCapture()
+      : set_(hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess) {}
+  ~RelaxedCapture() {
+    if (set_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+  }
+  RelaxedCapture(const RelaxedCapture &) = delete;
+  RelaxedCapture &operator=(const RelaxedCapture &) = delete;
+
+ private:
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+  bool set_;
+};
+
 // Owning device allocation (hipMalloc). Move-only.
 class DevBuf {
  public:
