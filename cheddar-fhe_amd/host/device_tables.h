@@ -58,6 +58,15 @@ class DevBuf {
   }
   void Resize(size_t bytes);
   void Upload(const void *host, size_t bytes);
+  // the same in the order of stream s, which is waited for
+  template <typename T>
+  void UploadOn(hipStream_t s, const std::vector<T> &v) {
+    Resize(v.size() * sizeof(T));
+    HipCheck(hipMemcpyAsync(ptr_, v.data(), v.size() * sizeof(T),
+                            hipMemcpyHostToDevice, s),
+             "hipMemcpyAsync");
+    HipCheck(hipStreamSynchronize(s), "hipStreamSynchronize");
+  }
   template <typename T>
   void Upload(const std::vector<T> &v) {
     Resize(v.size() * sizeof(T));

@@ -420,8 +420,10 @@ const Encoder<uint32_t>::CrtTable &Encoder<uint32_t>::CrtOf(
                       primes[i]);
     icrt[i] = pm::invmod(prod, primes[i]);
   }
+  // on the caller's stream: a copy on the null stream would end a graph that
+  // another thread records
   CrtTable t;
-  t.icrt.Upload(icrt);
+  t.icrt.UploadOn(CurrentStream(), icrt);
   Words q{1};
   for (int j = 0; j < lp; j++) q = MulSmall(q, primes[j]);
   // sum < lp * Q < 2^32 * Q
@@ -439,7 +441,7 @@ const Encoder<uint32_t>::CrtTable &Encoder<uint32_t>::CrtOf(
     for (size_t i = 0; i < width; i++)
       table[(lp + 1) * width + i] =
           (q[i] >> 1) | (i + 1 < width ? q[i + 1] << 31 : 0);
-    t.table.Upload(table);
+    t.table.UploadOn(CurrentStream(), table);
     t.width = static_cast<int>(width);
   }
   return crt_.emplace(key, std::move(t)).first->second;

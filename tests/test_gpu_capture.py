@@ -1,6 +1,6 @@
 """Calls of one thread while another thread records a graph: a hoisted
-evaluation whose temporaries go beyond the context's arena for the first time
-succeeds and leaves the recording whole."""
+evaluation whose temporaries go beyond the context's arena for the first time,
+and the first decode of a level, succeed and leave the recording whole."""
 import threading
 
 import numpy as np
@@ -87,3 +87,19 @@ def test_added_chunk_beside_a_capture(chain):
     large[0].run(res, x, large[1], stream=side.cuda_stream)
     for t, w in zip(res, got):
         assert np.array_equal(host(t), w)
+
+def test_first_decode_beside_a_capture(chain):
+    import torch
+    chd, ctx, main, aux = chain
+    r = np.random.default_rng(0xCA99)
+    msg = r.normal(size=512) + 1j * r.normal(size=512)
+    pt = zeros(5, N)
+    stream = torch.cuda.Stream().cuda_stream
+    torch.cuda.synchronize()
+    slots = ctx.encode(4, 0, float(1 << 30), msg, pt, stream)
+    got = _beside_a_capture(
+        chd, main, "thread_local",
+        lambda: ctx.decode(4, float(1 << 30), slots, pt, stream))
+    assert np.abs(got - msg).max() < 1e-5
+    assert np.array_equal(ctx.decode(4, float(1 << 30), slots, pt, stream),
+                          got)
