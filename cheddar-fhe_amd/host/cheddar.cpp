@@ -132,41 +132,66 @@ Workspace::External::~External() {
   ws_->strict_ = false;
 }
 
-uint32_t *Workspace::Push(size_t words) {
-  const size_t w = (words + 63) & ~static_cast<size_t>(63);  // 256-byte steps
-  for (size_t i = cur_chunk_;; i++) {
-    if (i > 0 && strict_) return nullptr;
-    if (i == chunks_.size() && !AddChunk(w)) return nullptr;
-    Chunk &c = chunks_[i];
-    if (w > c.cap - c.top) continue;
-    cur_chunk_ = i;
-    uint32_t *p = c.base + c.top;
-    c.top += w;
-    return p;
-  }
-}
-
-// false where nothing may be allocated: the bound is reached, the memory is
-// not there, or the calling stream is being captured
-bool Workspace::AddChunk(size_t words) {
-  const size_t bytes = words * sizeof(uint32_t);
+namespace {
+// whether the calling stream is being captured (or may not even be asked)
+bool Capturing() {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (bytes > kMaxExtraBytes - extra_bytes_) return false;
   const hipError_t e = hipStreamIsCapturing(CurrentStream(), &st);
   if (e != hipSuccess) (void)hipGetLastError();  // not the next launch's
-  if (e != hipSuccess || st != hipStreamCaptureStatusNone) return false;
-  Chunk c;
+  return e != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+}  // namespace
+
+uint32_t *Workspace::Push(size_t words) {
+  const size_t w = (words + 63) & ~static_cast<size_t>(63);  // 256-byte steps
+  size_t i = cur_chunk_;
+  while (i < chunks_.size() && w > chunks_[i].cap - chunks_[i].top) {
+    if (strict_) return nullptr;
+    i++;
+  }
+  if (i > 0 && Capturing()) {
+    if (i == chunks_.size()) return nullptr;
+    chunks_[i].captured = true;
+  } else if (i == chunks_.size()) {
+    if (!AddChunk(w)) return nullptr;
+    i = chunks_.size() - 1;
+  }
+  Chunk &c = chunks_[i];
+  cur_chunk_ = i;
+  uint32_t *p = c.base + c.top;
+  c.top += w;
+  return p;
+}
+
+// A chunk of at least `words` words at the end of chunks_, in place of the
+// idle ones; false when the bound is reached or the memory is not there.
+bool Workspace::AddChunk(size_t words) {
+  // chunks behind the current one are idle; earlier users' work on them ends
+  // before this stream's (Enter)
+  size_t idle = 0, kept = extra_bytes_ / sizeof(uint32_t);
+  for (size_t i = cur_chunk_ + 1; i < chunks_.size(); i++)
+    if (!chunks_[i].captured) idle += chunks_[i].cap;
+  kept -= idle;
+  const size_t cap = std::max(words, idle);
+  if ((kept + cap) * sizeof(uint32_t) > kMaxExtraBytes) return false;
+  RelaxedCapture relaxed;
   try {
-    RelaxedCapture relaxed;
-    c.buf.Resize(bytes);
+    if (idle > 0) {
+      HipCheck(hipStreamSynchronize(CurrentStream()), "hipStreamSynchronize");
+      for (size_t i = chunks_.size() - 1; i > cur_chunk_; i--)
+        if (!chunks_[i].captured) chunks_.erase(chunks_.begin() + i);
+      extra_bytes_ = kept * sizeof(uint32_t);
+    }
+    Chunk c;
+    c.buf.Resize(cap * sizeof(uint32_t));
+    c.base = c.buf.as<uint32_t>();
+    c.cap = cap;
+    chunks_.push_back(std::move(c));
   } catch (const std::exception &) {
-    (void)hipGetLastError();
+    (void)hipGetLastError();  // not the next launch's failure
     return false;
   }
-  c.base = c.buf.as<uint32_t>();
-  c.cap = words;
-  extra_bytes_ += bytes;
-  chunks_.push_back(std::move(c));
+  extra_bytes_ += cap * sizeof(uint32_t);
   return true;
 }
 

@@ -303,11 +303,14 @@ void CopyDeviceToDevice(DeviceVector<word> &dst,
 // one stream at a time: a call on a different stream than the previous call
 // first makes its stream wait for the event recorded at the end of that call.
 // Calls from several host threads are serialised by a mutex.
-// A call that needs more than the arena adds a chunk, which stays (at most
-// kMaxExtraBytes of them): stream-ordered memory goes back to the system at
-// the next synchronisation and is mapped again by the next call (a hoisted
-// 28 x 28 step transform, 0.8 GiB, 1.2 ms of 4.2 per call between
-// synchronisations).
+// A call that needs more than the arena adds a chunk, which stays with the
+// context: stream-ordered memory goes back to the system at the next
+// synchronisation and is mapped again by the next call (a hoisted 28 x 28 step
+// transform, 0.8 GiB, 1.2 ms of 4.2 per call between synchronisations). A
+// request that fits no chunk replaces the idle ones by one that holds them
+// all, so that what is served does not depend on the order of earlier calls.
+// Chunks take at most kMaxExtraBytes per context; beyond that a request is
+// stream-ordered.
 class Workspace {
  public:
   explicit Workspace(size_t words);
@@ -354,6 +357,8 @@ class Workspace {
     DevBuf buf;  // empty while External lends memory
     uint32_t *base = nullptr;
     size_t cap = 0, top = 0;  // words
+    // recorded into a graph, which goes on using it: never replaced
+    bool captured = false;
   };
   void Enter();
   void Leave() noexcept;

@@ -828,6 +828,39 @@ int main() {
                         "and single pass") + (centre ? ", centred" : ""), ok);
     }
   }
+  // temporaries beyond a workspace's arena: requests of many sizes leave no
+  // pieces that keep a later, larger one out of the bound, and memory that is
+  // in use stays where it is
+  {
+    constexpr size_t kMiB = (size_t{1} << 20) / sizeof(word);
+    Workspace ws(kMiB);
+    Workspace::Use use(&ws);
+    bool ok = true;
+    for (size_t mib : {200, 300, 400, 500, 600, 1800}) {
+      word *p = ws.Push(mib * kMiB);
+      ok = ok && p != nullptr;
+      if (p != nullptr) ws.Pop(p);
+    }
+    check("Workspace: one large request after several small ones", ok);
+    Workspace nested(kMiB);
+    Workspace::Use use2(&nested);
+    const std::vector<word> x = uniform(main_p, 1);
+    word *a1 = nested.Push(2 * kMiB), *a2 = nested.Push(64 * kMiB);
+    ok = a1 != nullptr && a2 != nullptr;
+    if (ok) {
+      upload(a1, x);
+      nested.Pop(a2);
+      word *a3 = nested.Push(128 * kMiB);  // more than a2's memory
+      ok = a3 != nullptr;
+      if (ok) {
+        upload(a3, uniform(main_p, 1));
+        ok = same(download(a1, kN), x);
+        nested.Pop(a3);
+      }
+      nested.Pop(a1);
+    }
+    check("Workspace: memory in use stays while idle memory is replaced", ok);
+  }
   // an invalid call throws cheddar::Error instead of exiting
   {
     bool threw = false;
