@@ -762,9 +762,10 @@ class Encoder<uint32_t> {
                   const NPInfo &np, double scale, const word *src) const;
 
  private:
+  struct Kept;
   // Pinned staging for one message (N / 2 complex values), which the kernels
   // read and write in place. Lent to one call, which synchronises its
-  // stream before giving it back; at most kKept stay with the encoder.
+  // stream before giving it back; at most kMaxStages stay with the encoder.
   class Stage {
    public:
     explicit Stage(const Encoder &enc);
@@ -775,22 +776,29 @@ class Encoder<uint32_t> {
     void Synchronize();
 
    private:
-    const Encoder &enc_;
+    Kept &kept_;
     double *p_ = nullptr;
     bool idle_ = false;
   };
-  static constexpr size_t kKept = 4;
-  struct StagePool {
-    std::mutex mu;
-    std::vector<double *> free;
-    ~StagePool();
-  };
-  mutable StagePool stages_;
+  static constexpr size_t kMaxStages = 4;
   // CRT constants of one prime set: (N prod_{k != i} q_k)^-1 mod q_i, then
   // chd_k_decode's table
   struct CrtTable {
     DevBuf icrt, table;
     int width = 0;  // 0: more words than the device decoder takes
+  };
+  // what an encoder keeps for the device, one for all copies of it
+  struct Kept {
+    Kept() { stages.reserve(kMaxStages); }  // no allocation in ~Stage
+    ~Kept();
+    // per stage: twiddle j of the stage of stride s at s + j, inverse then
+    // forward (device, 32768 complex values each)
+    DevBuf stage_twiddle;
+    std::mutex stage_mu;
+    std::vector<double *> stages;
+    // built on first use of a level
+    std::mutex crt_mu;
+    std::map<std::pair<int, int>, CrtTable> crt;
   };
   const CrtTable &CrtOf(const NPInfo &np) const;
   void DecodeHost(std::vector<Complex> &message, const NPInfo &np, int slots,
@@ -799,12 +807,7 @@ class Encoder<uint32_t> {
   const NTTHandler<word> *ntt_handler_;
   const int m_;  // 2N
   std::vector<Complex> twiddle_;
-  // per stage: twiddle j of the stage of stride s at s + j, inverse then
-  // forward (device, 32768 complex values each)
-  DevBuf stage_twiddle_;
-  // built on first use of a level, kept with the encoder
-  mutable std::mutex crt_mu_;
-  mutable std::map<std::pair<int, int>, CrtTable> crt_;
+  std::shared_ptr<Kept> kept_;
 };
 
 template <typename word>

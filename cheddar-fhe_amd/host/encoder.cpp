@@ -166,30 +166,34 @@ Encoder<uint32_t>::Encoder(const Parameter<word> &param,
       tw[half + s + j] = twiddle_[r * gap];
     }
   }
-  stage_twiddle_.Upload(tw);
+  kept_->stage_twiddle.Upload(tw);
 }
 
 Encoder<uint32_t>::Encoder(const Parameter<word> &param)
-    : param_(param), ntt_handler_(nullptr), m_(2 * param.degree_), twiddle_(m_) {
+    : param_(param),
+      ntt_handler_(nullptr),
+      m_(2 * param.degree_),
+      twiddle_(m_),
+      kept_(std::make_shared<Kept>()) {
   for (int i = 0; i < m_; i++)
     twiddle_[i] = std::polar(1.0, 2.0 * M_PI * i / m_);
 }
 
-Encoder<uint32_t>::StagePool::~StagePool() {
-  for (double *p : free) (void)hipHostFree(p);
+Encoder<uint32_t>::Kept::~Kept() {
+  for (double *p : stages) (void)hipHostFree(p);
 }
 
-Encoder<uint32_t>::Stage::Stage(const Encoder &enc) : enc_(enc) {
+Encoder<uint32_t>::Stage::Stage(const Encoder &enc) : kept_(*enc.kept_) {
   {
-    std::lock_guard<std::mutex> lock(enc_.stages_.mu);
-    if (!enc_.stages_.free.empty()) {
-      p_ = enc_.stages_.free.back();
-      enc_.stages_.free.pop_back();
+    std::lock_guard<std::mutex> lock(kept_.stage_mu);
+    if (!kept_.stages.empty()) {
+      p_ = kept_.stages.back();
+      kept_.stages.pop_back();
       return;
     }
   }
   HipCheck(hipHostMalloc(reinterpret_cast<void **>(&p_),
-                         enc_.param_.degree_ * sizeof(double),
+                         enc.param_.degree_ * sizeof(double),
                          hipHostMallocDefault),
            "hipHostMalloc");
 }
@@ -202,9 +206,9 @@ void Encoder<uint32_t>::Stage::Synchronize() {
 Encoder<uint32_t>::Stage::~Stage() {
   // a call that ended early may have kernels on the buffer
   if (!idle_) (void)hipStreamSynchronize(CurrentStream());
-  std::lock_guard<std::mutex> lock(enc_.stages_.mu);
-  if (enc_.stages_.free.size() < kKept)
-    enc_.stages_.free.push_back(p_);
+  std::lock_guard<std::mutex> lock(kept_.stage_mu);
+  if (kept_.stages.size() < kMaxStages)
+    kept_.stages.push_back(p_);
   else
     (void)hipHostFree(p_);
 }
@@ -331,7 +335,7 @@ int Encoder<uint32_t>::EncodeTo(word *dst, int level, double scale,
     double *coef = work + 2 * slots;
     K(chd_k_encode_coefficients(coef, work, msg, msg + (inter ? 1 : len),
                                 stride, len, log_slots, scale,
-                                stage_twiddle_.as<const double>(),
+                                kept_->stage_twiddle.as<const double>(),
                                 CurrentStream()));
     const chd_limb_map m = ntt_handler_->LimbMapOf(np);
     K(chd_k_encode_residues(&ntt_handler_->Tables(), &m,
@@ -405,10 +409,10 @@ void Encoder<uint32_t>::EncodeConstant(Constant<word> &constant, int level,
 // and the words of Q / q_j, Q and floor(Q / 2)
 const Encoder<uint32_t>::CrtTable &Encoder<uint32_t>::CrtOf(
     const NPInfo &np) const {
-  std::lock_guard<std::mutex> lock(crt_mu_);
+  std::lock_guard<std::mutex> lock(kept_->crt_mu);
   const auto key = std::make_pair(np.num_main_, np.num_ter_);
-  const auto it = crt_.find(key);
-  if (it != crt_.end()) return it->second;
+  const auto it = kept_->crt.find(key);
+  if (it != kept_->crt.end()) return it->second;
   const std::vector<word> primes = param_.GetPrimeVector(np);
   const int lp = static_cast<int>(primes.size());
   std::vector<word> icrt(lp);
@@ -444,7 +448,7 @@ const Encoder<uint32_t>::CrtTable &Encoder<uint32_t>::CrtOf(
     t.table.UploadOn(CurrentStream(), table);
     t.width = static_cast<int>(width);
   }
-  return crt_.emplace(key, std::move(t)).first->second;
+  return kept_->crt.emplace(key, std::move(t)).first->second;
 }
 
 // Encode.cpp:45-82 and 192-246 (PlaintextToComplexVector)
@@ -488,7 +492,7 @@ void Encoder<uint32_t>::DecodeFrom(double *re, double *im, int stride,
     K(chd_k_decode(out, out + (inter ? 1 : slots), stride, work,
                    tmp.mx_.data(), lp, crt.table.as<const word>(), crt.width,
                    Log2CeilInt(slots), scale,
-                   stage_twiddle_.as<const double>() + n, CurrentStream()));
+                   kept_->stage_twiddle.as<const double>() + n, CurrentStream()));
     stage.Synchronize();
     if (inter) {
       (void)CopyChecked(re, out, 2 * slots, &finite);

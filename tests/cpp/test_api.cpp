@@ -490,6 +490,19 @@ int main() {
       err = std::max(err, std::abs(back[i] - msg[i]));
     check("Encoder Encode/Decode round trip",
           pt.GetNumSlots() == (1 << 12) && pt.GetNP() == np && err < 1e-3);
+    // a copy, which shares what the encoder keeps on the device
+    bool copied = false;
+    {
+      const Encoder<word> copy(ctx->encoder_);
+      Plaintext<word> pt2;
+      copy.Encode(pt2, L - 1, 0x1p30, msg);
+      std::vector<Complex> back2;
+      copy.Decode(back2, pt2);
+      copied = same(download(pt2.mx_.data(), qw), download(pt.mx_.data(), qw)) &&
+               back2 == back;
+    }
+    ctx->encoder_.Decode(back, pt);
+    check("Encoder copy", copied && std::abs(back[0] - msg[0]) < 1e-3);
     Constant<word> c;
     ctx->encoder_.EncodeConstant(c, 3, 0x1p20, -1.5);
     std::vector<word> cx = download(c.cx_.data(), c.cx_.size());
