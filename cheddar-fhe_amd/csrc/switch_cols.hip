@@ -9,10 +9,11 @@
 // inverse row pass to the forward row pass through LDS instead of two passes
 // over memory between three launches.
 //
-// Data between the row passes and this kernel is column-blocked: word
-//   ((col >> 2) * 256 + row) * 4 + (col & 3)
-// of a limb. A row pass's 16-row tile is then 64 pieces of 256 contiguous
-// bytes, and four columns are 4 KiB contiguous, whatever the tile width here.
+// Data between the row passes and this kernel is column-blocked: index
+// row * 256 + col of a limb is word
+//   ((col >> 2) * 256 + 16 * (row % 16) + row / 16) * 4 + (col & 3).
+// A row pass's tile t, rows 16 r + t, is then 64 pieces of 256 contiguous bytes,
+// and four columns are 4 KiB contiguous, whatever the tile width here.
 //
 // Work split. A workgroup (8 waves) owns kW = 2 columns of one job and all (or a
 // 16-aligned part of) its destinations. A wave works on 4 / kW limbs at a

@@ -176,7 +176,7 @@ int chd_k_bconv_batch(const chd_tables *t, const chd_limb_map *m,
 /* A base switch (ModUp, ModDown, Rescale) as three launches: the inverse row
  * pass, the column stage, the forward row pass. Between them limbs are
  * column-blocked: index row * 256 + col of a limb sits at word
- * ((col >> 2) * 256 + row) * 4 + (col & 3), unreduced.
+ * ((col >> 2) * 256 + 16 * (row % 16) + row / 16) * 4 + (col & 3), unreduced.
  *
  * chd_k_ntt_inv_rows: the first pass (stages 15..8) of chd_k_ntt_inv, or of
  * chd_k_ntt_inv_mul when src_mul is given, into column-blocked dst, which
