@@ -351,40 +351,6 @@ int Encoder<uint32_t>::EncodeTo(word *dst, int level, double scale,
   return slots;
 }
 
-std::vector<Complex> Encoder<uint32_t>::PadToPowerOfTwo(
-    const std::vector<Complex> &message) {
-  const int len = static_cast<int>(message.size());
-  std::vector<Complex> padded(static_cast<size_t>(1) << Log2CeilInt(len));
-  std::copy(message.begin(), message.end(), padded.begin());
-  return padded;
-}
-
-// the device half of Encode: upload the residues, NTT with Montgomery
-// conversion
-void Encoder<uint32_t>::EncodeResidues(Plaintext<word> &ptxt, int level,
-                                       double scale, int slots,
-                                       const std::vector<word> &mx,
-                                       int num_aux) const {
-  AssertTrue(ntt_handler_ != nullptr, "Encode: host-only encoder");
-  const NPInfo np = param_.LevelToNP(level, num_aux);
-  AssertTrue(mx.size() == static_cast<size_t>(np.GetNumTotal()) *
-                              static_cast<size_t>(param_.degree_),
-             "Encode: residues do not match the level");
-  Plaintext<word> out(np, param_.degree_);
-  HipCheck(hipMemcpyAsync(out.mx_.data(), mx.data(), mx.size() * sizeof(word),
-                          hipMemcpyHostToDevice, CurrentStream()),
-           "hipMemcpyAsync");
-  // the aux limbs follow the q limbs directly: views with their aux size
-  const int aux_words = num_aux * param_.degree_;
-  DvView<word> v = out.mx_.View(aux_words);
-  ntt_handler_->NTT(v, np, out.mx_.ConstView(aux_words), true);
-  // mx is the caller's host memory: the copy has to finish before it goes
-  HipCheck(hipStreamSynchronize(CurrentStream()), "hipStreamSynchronize");
-  out.SetNumSlots(slots);
-  out.SetScale(scale);
-  ptxt = std::move(out);
-}
-
 // Encode.cpp:248-273
 void Encoder<uint32_t>::EncodeConstant(Constant<word> &constant, int level,
                                        double scale, double number,
