@@ -1983,8 +1983,9 @@ hipError_t launch_ntt_fwd(const NttArgs &a, int num_limbs, int num_polys,
   // passes, spread over small workgroups, grow with the limbs: 11.6, 12.1,
   // 14.6, 17.9, 23.7, 26.0 (12.3, 12.9, 15.7, 18.1, 23.1, 25.5). So two passes
   // up to half a round and up to a quarter of the second; later rounds hide
-  // it (144 limbs 35.5 against 38.0 us). The ModDown epilogue keeps the
-  // single pass: its caller makes that choice.
+  // it (144 limbs 35.5 against 38.0 us). Above 2^30 the lines would lie at 40
+  // and above 96 limbs, where one rule for both kinds costs 0.5 and 2 us. The
+  // ModDown epilogue keeps the single pass: its caller makes that choice.
   const int items = num_limbs * num_polys;
   const bool one_pass = items > 32 && (items <= 64 || items > 80);
   if (a.src_disjoint && !a.fwd_two_pass &&

@@ -24,9 +24,10 @@
 //
 // Why this shape. The launch it replaces three of moved 56 MiB (ModUp) and 35
 // MiB (merged ModDown) of a 24 + 8 limb, dnum 3 key switch between memory and
-// the CUs; this one moves 24 and 16 MiB and is bound by VALU issue (4.8 and
-// 3.6 M wave instructions, 8.9 and 6.7 us of it spread evenly) and by the
-// latency of its three phases at two waves per SIMD: 20.0 and 15.2 us
+// the CUs; this one moves 24 and 16 MiB and is bound by the latency of its
+// three phases at two to three waves per SIMD (26-28 % VALU-busy; its 4.6 and
+// 3.4 M wave instructions are 7.4 and 5.6 us spread evenly; the 24 jobs of a
+// hoisted batch keep the VALU 63 % busy): 20.0 and 15.2 us
 // against 29.4 us (inverse columns + BConv + forward columns) and, with the
 // row pass that follows, 25 against 31.7 us (inverse columns + BConv +
 // single-pass NTT). One 24-limb product with merged rescale went from 89.3 to

@@ -253,8 +253,10 @@ int chd_hoist_baby_steps(const chd_context *ctx, int level,
  * from its plaintexts, then evaluated many times): chd_hoist_create copies
  * the plaintexts (layout as for chd_hoist_evaluate) and synchronises the
  * stream; chd_hoist_run evaluates one ciphertext at the handler's level,
- * reusing the handler's baby-step and result buffers (no allocation after
- * the first run; runs of one handler must not overlap). */
+ * reusing the handler's baby-step buffers and reading and writing the
+ * caller's (no allocation after the first run; runs of one handler must not
+ * overlap). Plaintext words are canonical residues; with at most 8 giant
+ * steps representatives in (-q, q), as signed integers, do as well. */
 typedef struct chd_hoist chd_hoist;
 int chd_hoist_create(chd_hoist **out, const chd_context *ctx, int level,
                      int num_gs, const int *gs, int num_bs, const int *bs,

@@ -94,7 +94,7 @@ def test_ntt_forward_two_pass_config2(chd):
 def test_ntt_inverse_single_pass(chd, bits):
     """the single-pass inverse over residue classes (chd_ntt_inverse_single_
     pass) at the config-2 shape, on 30-bit primes (lazy butterflies) and
-    31-bit primes (reference-form butterflies), both epilogue constants,
+    31-bit primes (both inputs reduced), both epilogue constants,
     against the oracle; an overlapping destination is refused"""
     primes = (Q30 if bits == 30 else Q31)[:32]
     plan = chd.NttPlan(primes)
@@ -117,8 +117,8 @@ def test_ntt_inverse_single_pass(chd, bits):
 
 
 def test_ntt_31bit_primes_batch(chd):
-    """the config-2 batch shape on 31-bit primes (the reference-form
-    butterflies of every kernel) against the oracle, both directions"""
+    """the config-2 batch shape on 31-bit primes (the reduced butterflies of
+    every kernel) against the oracle, both directions"""
     primes = Q31[:32]
     plan = chd.NttPlan(primes)
     x = np.stack([uniform_limbs(rng(950 + p), primes) for p in range(2)])
